@@ -24,9 +24,11 @@
 //    RNE_e4m3fn(clamp(x / scale, +-448)) via v_cvt_pk_fp8_f32 (one dword per
 //    lane); 16-bit caches take the dtype value (8 bytes per lane).
 //
-//  kv_amax<T> + kv_scales_finalize   one workgroup per (KV head, K or V)
-//    scans every token (no atomics, deterministic), then one workgroup turns
-//    the maxima into scales.
+//  kv_amax8<T, CS>   the fp8 cache scales, fast path (the layouts of
+//    kv_rope_write8): workgroups of 16 waves over chunks of tokens, all heads,
+//    K and V read once in whole rows; a workgroup folds its maxima in LDS and
+//    combines its scales by atomic maximum (a maximum has no order: the result
+//    is deterministic).  kv_amax<T>: the general path, by (head, K or V, chunk).
 //
 // Reference semantics (paths relative to the reference repo root):
 //   integrations/vllm/l20_rope_kv.py:26-137 (interleaved), :140-253 (neox),
@@ -168,30 +170,86 @@ template <typename T> __device__ __forceinline__ i32x4 pack8(const float (&x)[8]
   const i32x2 a = pack4<T>(lo), b = pack4<T>(hi);
   return i32x4{a[0], a[1], b[0], b[1]};
 }
-// n (4 or 8) consecutive cos/sin values from a table of CS type (0 bf16, 1 fp16, 2 fp32).
-template <int CS, int N> __device__ __forceinline__ void load_cs(const void *base, int64_t off, float (&c)[8]) {
+// The cos and sin of one row's eight dims as loaded (table type CS: 0 bf16, 1
+// fp16, 2 fp32), unpacked where they are used: eight consecutive values each
+// for a neox pair layout, four (one per pair) for an interleaved one.  Kept as
+// loaded, 16-bit tables take 8 registers a row and not 16 (kv_rope_write8 on a
+// 16K-token chunk, 32 heads of 128: 65.5 -> 63.2 us).
+template <int CS> struct CosSin {
+  i32x4 c[CS == 2 ? 2 : 1], s[CS == 2 ? 2 : 1];
+};
+template <int CS, int N>
+__device__ __forceinline__ void load_cs(const void *base, int64_t off, i32x4 (&w)[CS == 2 ? 2 : 1]) {
   if constexpr (CS == 2) {
-    const float *src = reinterpret_cast<const float *>(base) + off;
-    const f32x4 a = *reinterpret_cast<const f32x4 *>(src);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) c[i] = a[i];
-    if constexpr (N == 8) {
-      const f32x4 b = *reinterpret_cast<const f32x4 *>(src + 4);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[4 + i] = b[i];
-    }
+    const i32x4 *src = reinterpret_cast<const i32x4 *>(reinterpret_cast<const float *>(base) + off);
+    w[0] = src[0];
+    if constexpr (N == 8) w[1] = src[1];
   } else {
-    typedef typename std::conditional<CS == 0, __bf16, _Float16>::type E;
-    const E *src = reinterpret_cast<const E *>(base) + off;
+    const uint16_t *src = reinterpret_cast<const uint16_t *>(base) + off;
     if constexpr (N == 8) {
-      unpack8<E>(*reinterpret_cast<const i32x4 *>(src), c);
+      w[0] = *reinterpret_cast<const i32x4 *>(src);
     } else {
-      float q[4];
-      load4(src, q);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) c[i] = q[i];
+      const i32x2 v = *reinterpret_cast<const i32x2 *>(src);
+      w[0] = i32x4{v[0], v[1], 0, 0};
     }
   }
+}
+// dims [e0, e0 + 8) (e0 < rot) of the row at `pos`
+template <int CS>
+__device__ __forceinline__ void load_row_cs(const Params &p, int64_t pos, int e0, int half, CosSin<CS> &w) {
+  const int64_t base = pos * p.cs_sp;
+  if (p.neox) {
+    const int t0 = e0 < half ? e0 : e0 - half;
+    load_cs<CS, 8>(p.cs, base + t0, w.c);
+    load_cs<CS, 8>(p.cs, base + half + t0, w.s);
+  } else {
+    load_cs<CS, 4>(p.cs, base + (e0 >> 1), w.c);
+    load_cs<CS, 4>(p.cs, base + half + (e0 >> 1), w.s);
+  }
+}
+template <int CS> __device__ __forceinline__ void unpack_cs(const i32x4 (&w)[CS == 2 ? 2 : 1], float (&x)[8]) {
+  if constexpr (CS == 2) {
+    const f32x4 a = __builtin_bit_cast(f32x4, w[0]), b = __builtin_bit_cast(f32x4, w[1]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[i] = a[i];
+      x[4 + i] = b[i];
+    }
+  } else if constexpr (CS == 1) {
+    unpack8<_Float16>(w[0], x);
+  } else {
+    unpack8<__bf16>(w[0], x);
+  }
+}
+
+// Rotate eight dims x in place; pw holds the neox partner's eight dims, first
+// says that x is in the first half of the rotary dims.
+template <typename T, int CS>
+__device__ __forceinline__ void rotate8(const Params &p, float (&x)[8], i32x4 pw, const CosSin<CS> &w, bool first) {
+#pragma clang fp contract(off)
+  float y[8], c[8], sn[8];
+  unpack_cs<CS>(w.c, c);
+  unpack_cs<CS>(w.s, sn);
+  if (p.neox) {
+    float pr[8];
+    unpack8<T>(pw, pr);
+    const float sg = first ? -1.0f : 1.0f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float a = x[i] * c[i];
+      const float b = (pr[i] * sn[i]) * sg;
+      y[i] = a + b;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float a = x[i] * c[i >> 1];
+      const float b = (x[i ^ 1] * sn[i >> 1]) * ((i & 1) ? 1.0f : -1.0f);
+      y[i] = a + b;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i] = y[i];
 }
 
 // Four values -> four e4m3fn codes in one dword: RNE of clamp(x / scale).
@@ -261,20 +319,10 @@ __global__ __launch_bounds__(256) void kv_rope_write8(Params p, int64_t rows_q, 
     head[u] = h;
   }
   // ---- cos / sin of the lanes' dims ----
-  float c[kRowsPerLane][8], sn[kRowsPerLane][8];
+  CosSin<CS> cs[kRowsPerLane];
 #pragma unroll
   for (int u = 0; u < kRowsPerLane; ++u) {
-    if (live[u] && rot_lane) {
-      const int64_t base = pos[u] * p.cs_sp;
-      if (p.neox) {
-        const int t0 = e0 < half ? e0 : e0 - half;
-        load_cs<CS, 8>(p.cs, base + t0, c[u]);
-        load_cs<CS, 8>(p.cs, base + half + t0, sn[u]);
-      } else {
-        load_cs<CS, 4>(p.cs, base + (e0 >> 1), c[u]);
-        load_cs<CS, 4>(p.cs, base + half + (e0 >> 1), sn[u]);
-      }
-    }
+    if (live[u] && rot_lane) load_row_cs<CS>(p, pos[u], e0, half, cs[u]);
   }
   // ---- rotate, store back, write the caches ----
 #pragma unroll
@@ -287,29 +335,7 @@ __global__ __launch_bounds__(256) void kv_rope_write8(Params p, int64_t rows_q, 
     if (!live[u]) continue;
     float x[8];
     unpack8<T>(xw[u], x);
-    if (rot_lane) {
-      float y[8];
-      if (p.neox) {
-        float pr[8];
-        unpack8<T>(pw, pr);
-        const float sg = e0 < half ? -1.0f : 1.0f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float a = x[i] * c[u][i];
-          const float b = (pr[i] * sn[u][i]) * sg;
-          y[i] = a + b;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float a = x[i] * c[u][i >> 1];
-          const float b = (x[i ^ 1] * sn[u][i >> 1]) * ((i & 1) ? 1.0f : -1.0f);
-          y[i] = a + b;
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = y[i];
-    }
+    if (rot_lane) rotate8<T, CS>(p, x, pw, cs[u], e0 < half);
     const i32x4 out = pack8<T>(x);
     __builtin_nontemporal_store(out, reinterpret_cast<i32x4 *>(row[u] + e0));
     if (!is_k[u]) continue;
@@ -376,29 +402,175 @@ __global__ __launch_bounds__(256) void kv_rope_write(Params p) {
   }
 }
 
-// amax of the stored K (rotated, dtype-rounded) or of V over all tokens of
-// one KV head: workgroup (h, which), 1024 threads, token-strided.
+// ---------------------------------------------------------------------------
+// fp8 cache scales
+// ---------------------------------------------------------------------------
+// max(amax / 448, 1e-12).  Correctly rounded division is monotone, so the
+// maximum of the workgroups' scales is the scale of the overall maximum: the
+// workgroups combine scales, and no pass over the maxima follows.
+__device__ __forceinline__ float scale_of(float amax) { return fmaxf(__fdiv_rn(amax, kFp8Max), 1e-12f); }
+
+constexpr int kScaleThreads = 1024;
+constexpr int kScaleMaxGroups = kScaleThreads / 4;  // lane groups of a workgroup at the smallest head_dim (32)
+// Rows per lane in flight (fp32 tables take twice the registers).
+constexpr int scale_rows(int cs) { return cs == 2 ? 2 : 4; }
+
+// Every scale to its lower bound, ahead of the workgroups' atomic maxima.
+__global__ void kv_scales_init(float *k_scales, float *v_scales, int hkv) {
+  const int h = blockIdx.x * blockDim.x + threadIdx.x;
+  if (h < hkv) k_scales[h] = v_scales[h] = 1e-12f;
+}
+
+// One workgroup's maxima -> the scales.  A positive float orders as its bits.
+// single: the only workgroup of the call, which stores (no kv_scales_init ran).
+// All of a workgroup's K (V) atomics leave in one instruction over consecutive
+// words: device-scope atomics on one line are served one request at a time.
+__device__ __forceinline__ void publish_scale(float *out, int h, float amax, bool single) {
+  const float s = scale_of(amax);
+  if (single) out[h] = s;
+  else atomicMax(reinterpret_cast<unsigned int *>(out) + h, __builtin_bit_cast(unsigned int, s));
+}
+
+// The fast path: amax of the stored K (rotated, dtype-rounded) and V of a chunk
+// of tokens, every head.  HBM-bound: K and V are read once, in whole rows (a
+// lane owns eight contiguous dims, D/8 lanes a row, scale_rows rows of K and
+// V in flight per lane), and every lane group keeps one head, so the maxima stay
+// in registers until the workgroup's LDS fold.  blockIdx.y: block of hb heads.
+// 16K tokens of 4 KV heads at head_dim 128 (38 MB): 13.5 us, 2.8 TB/s, where one
+// workgroup per (head, K or V) took 3158 us.  256 workgroups of 16 waves, the
+// whole chunk in flight at once; 1024 of 4 waves 22.3 us per call and 512 of 8
+// 17.0 us (more atomics on one line), against 15.1 us; without the atomics 13.2.
+template <typename T, int CS>
+__global__ __launch_bounds__(kScaleThreads) void kv_amax8(Params p, float *k_out, float *v_out, int hb, int chunk,
+                                                         int per_head, int single) {
+#pragma clang fp contract(off)
+  constexpr int kRows = scale_rows(CS);
+  __shared__ float s_max[2][kScaleMaxGroups];
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int lpr = p.d >> 3;     // lanes per row
+  const int rpw = 64 / lpr;     // rows per wave and pass
+  const int g = lane / lpr;
+  const int l = lane - g * lpr;
+  const int e0 = 8 * l;
+  const int half = p.rot >> 1;
+  const bool rot_lane = e0 < p.rot;
+  const int tpp = (kScaleThreads / 64) * rpw / hb;  // tokens per pass
+  const int group = wave * rpw + g;
+  const int off = group / hb;  // the group's token of a pass
+  const int head = blockIdx.y * hb + (group - off * hb);
+  const bool used = g < rpw && off < tpp && head < p.hkv;
+  const int64_t t_end = min((int64_t)p.tokens, ((int64_t)blockIdx.x + 1) * chunk);
+  const T *kbase = reinterpret_cast<const T *>(p.k) + (int64_t)head * p.k_sh + e0;
+  const T *vbase = reinterpret_cast<const T *>(p.v) + (int64_t)head * p.v_sh + e0;
+  // the neox partner's words, from the lane half/8 away in the same row
+  const int src = (p.neox && rot_lane) ? g * lpr + (e0 < half ? l + (half >> 3) : l - (half >> 3)) : lane;
+  float mk = 0.0f, mv = 0.0f;
+  for (int64_t t0 = (int64_t)blockIdx.x * chunk; t0 < t_end; t0 += kRows * tpp) {  // uniform: every lane shuffles
+    i32x4 kw[kRows], vw[kRows];
+    int64_t pos[kRows];
+    bool live[kRows];
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int64_t t = t0 + (int64_t)u * tpp + off;
+      live[u] = used && t < t_end;
+      kw[u] = vw[u] = i32x4{0, 0, 0, 0};
+      pos[u] = 0;
+      if (live[u]) {
+        kw[u] = *reinterpret_cast<const i32x4 *>(kbase + t * p.k_st);
+        vw[u] = *reinterpret_cast<const i32x4 *>(vbase + t * p.v_st);
+        pos[u] = p.pos[t];
+        const int64_t slot = p.slots[t];
+        live[u] = slot >= 0 && (slot >> 4) < p.num_pages;  // else not stored
+      }
+    }
+    CosSin<CS> cs[kRows];
+#pragma unroll
+    for (int u = 0; u < kRows; ++u)
+      if (live[u] && rot_lane) load_row_cs<CS>(p, pos[u], e0, half, cs[u]);
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      i32x4 pw;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pw[i] = __shfl(kw[u][i], src);
+      if (!live[u]) continue;
+      float x[8];
+      unpack8<T>(kw[u], x);
+      if (rot_lane) rotate8<T, CS>(p, x, pw, cs[u], e0 < half);
+      unpack8<T>(pack8<T>(x), x);  // the stored model-dtype values
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mk = fmaxf(mk, fabsf(x[i]));
+      unpack8<T>(vw[u], x);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mv = fmaxf(mv, fabsf(x[i]));
+    }
+  }
+  // the row's lanes
+  float rk = mk, rv = mv;
+  if ((lpr & (lpr - 1)) == 0) {
+    for (int o = 1; o < lpr; o <<= 1) {
+      rk = fmaxf(rk, __shfl_xor(rk, o));
+      rv = fmaxf(rv, __shfl_xor(rv, o));
+    }
+  } else {  // head_dim 96: 12 lanes
+    for (int i = 0; i < lpr; ++i) {
+      rk = fmaxf(rk, __shfl(mk, min(g * lpr + i, 63)));
+      rv = fmaxf(rv, __shfl(mv, min(g * lpr + i, 63)));
+    }
+  }
+  if (l == 0 && g < rpw) {
+    s_max[0][group] = used ? rk : 0.0f;
+    s_max[1][group] = used ? rv : 0.0f;
+  }
+  __syncthreads();
+  const int groups = (kScaleThreads / 64) * rpw;
+  if (per_head) {
+    const int i = threadIdx.x;  // head i of the block
+    if (i >= hb || blockIdx.y * hb + i >= p.hkv) return;
+    float k = 0.0f, v = 0.0f;
+    for (int o = 0; o < tpp; ++o) {
+      k = fmaxf(k, s_max[0][o * hb + i]);
+      v = fmaxf(v, s_max[1][o * hb + i]);
+    }
+    publish_scale(k_out, blockIdx.y * hb + i, k, single);
+    publish_scale(v_out, blockIdx.y * hb + i, v, single);
+  } else {
+    float k = 0.0f, v = 0.0f;  // the maximum over heads, in every entry
+    for (int o = 0; o < groups; ++o) {
+      k = fmaxf(k, s_max[0][o]);
+      v = fmaxf(v, s_max[1][o]);
+    }
+    for (int h = threadIdx.x; h < p.hkv; h += kScaleThreads) {
+      publish_scale(k_out, h, k, single);
+      publish_scale(v_out, h, v, single);
+    }
+  }
+}
+
+// The general path (any layout the checks accept): workgroup (h, K or V, chunk
+// of tokens), 16 waves over the chunk's tokens, four dims per lane.
 template <typename T>
-__global__ __launch_bounds__(1024) void kv_amax(Params p, float *k_out, float *v_out) {
+__global__ __launch_bounds__(1024) void kv_amax(Params p, float *k_out, float *v_out, int chunk, int per_head) {
   __shared__ float s_red[16];
   const int h = blockIdx.x;
   const bool is_k = blockIdx.y == 0;
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
   const int e0 = 4 * lane;
+  const int64_t t_end = min((int64_t)p.tokens, ((int64_t)blockIdx.z + 1) * chunk);
   float m = 0.0f;
   if (e0 < p.d) {
-    for (int t = wave; t < p.tokens; t += 16) {
+    for (int64_t t = (int64_t)blockIdx.z * chunk + wave; t < t_end; t += 16) {
       const int64_t slot = p.slots[t];
       if (slot < 0 || (slot >> 4) >= p.num_pages) continue;  // not stored
       float x[4];
       if (is_k) {
-        const T *row = reinterpret_cast<const T *>(p.k) + (int64_t)t * p.k_st + (int64_t)h * p.k_sh;
+        const T *row = reinterpret_cast<const T *>(p.k) + t * p.k_st + (int64_t)h * p.k_sh;
         rope4<T>(p, row, p.pos[t], e0, x);
         const i32x2 w = pack4<T>(x);
         unpack4<T>(w, x);
       } else {
-        load4(reinterpret_cast<const T *>(p.v) + (int64_t)t * p.v_st + (int64_t)h * p.v_sh + e0, x);
+        load4(reinterpret_cast<const T *>(p.v) + t * p.v_st + (int64_t)h * p.v_sh + e0, x);
       }
 #pragma unroll
       for (int i = 0; i < 4; ++i) m = fmaxf(m, fabsf(x[i]));
@@ -408,20 +580,14 @@ __global__ __launch_bounds__(1024) void kv_amax(Params p, float *k_out, float *v
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
   if (lane == 0) s_red[wave] = m;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    float r = 0.0f;
-    for (int w = 0; w < 16; ++w) r = fmaxf(r, s_red[w]);
-    (is_k ? k_out : v_out)[h] = r;
+  float r = 0.0f;
+  for (int w = 0; w < 16; ++w) r = fmaxf(r, s_red[w]);
+  float *out = is_k ? k_out : v_out;
+  if (per_head) {
+    if (threadIdx.x == 0) publish_scale(out, h, r, false);
+  } else {
+    for (int i = threadIdx.x; i < p.hkv; i += 1024) publish_scale(out, i, r, false);
   }
-}
-
-// amax -> max(amax / 448, 1e-12), per head or (per_head = 0) the maximum over heads.
-__global__ void kv_scales_finalize(float *k_scales, float *v_scales, int hkv, int per_head) {
-  if (threadIdx.x >= 2) return;
-  float *s = threadIdx.x == 0 ? k_scales : v_scales;
-  float all = 0.0f;
-  for (int h = 0; h < hkv; ++h) all = fmaxf(all, s[h]);
-  for (int h = 0; h < hkv; ++h) s[h] = fmaxf(__fdiv_rn(per_head ? s[h] : all, kFp8Max), 1e-12f);
 }
 
 }  // namespace l20kv
@@ -549,6 +715,18 @@ void launch_fast(const l20kv::Params &p, int cs_dtype, int64_t rows_q, int64_t r
     hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0>), grid, dim3(256), 0, s, p, rows_q, rows_all);
 }
 
+template <typename T>
+void launch_amax8(const l20kv::Params &p, dim3 grid, float *k_scales, float *v_scales, int hb, int chunk, int per_head,
+                  bool single, hipStream_t s) {
+  const dim3 block(l20kv::kScaleThreads);
+  if (p.cs_dtype == 2)
+    hipLaunchKernelGGL((l20kv::kv_amax8<T, 2>), grid, block, 0, s, p, k_scales, v_scales, hb, chunk, per_head, single);
+  else if (p.cs_dtype == 1)
+    hipLaunchKernelGGL((l20kv::kv_amax8<T, 1>), grid, block, 0, s, p, k_scales, v_scales, hb, chunk, per_head, single);
+  else
+    hipLaunchKernelGGL((l20kv::kv_amax8<T, 0>), grid, block, 0, s, p, k_scales, v_scales, hb, chunk, per_head, single);
+}
+
 int32_t launched() {
   const hipError_t e = hipGetLastError();
   if (e != hipSuccess) {
@@ -610,18 +788,47 @@ int32_t l20_pd_kv_fp8_scales(const l20_pd_kv_write_args *a, float *k_scales, flo
   const int32_t rc = check(a);
   if (rc != L20_PD_OK) return rc;
   if (!k_scales || !v_scales) return set_error(L20_PD_EINVAL, "null scale output");
-  const l20kv::Params p = params(*a);
+  l20_pd_kv_write_args b = *a;
+  b.query = nullptr;  // not read: its layout does not decide the path
+  const l20kv::Params p = params(b);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (a->dtype == L20_PD_BF16)
-    hipLaunchKernelGGL((l20kv::kv_amax<__bf16>), dim3((unsigned)a->num_kv_heads, 2), dim3(1024), 0, s, p, k_scales,
-                       v_scales);
-  else
-    hipLaunchKernelGGL((l20kv::kv_amax<_Float16>), dim3((unsigned)a->num_kv_heads, 2), dim3(1024), 0, s, p,
-                       k_scales, v_scales);
-  int32_t r = launched();
-  if (r != L20_PD_OK) return r;
-  hipLaunchKernelGGL(l20kv::kv_scales_finalize, dim3(1), dim3(64), 0, s, k_scales, v_scales, a->num_kv_heads,
-                     per_head);
+  const bool bf = a->dtype == L20_PD_BF16;
+  const int tokens = std::max(1, p.tokens);
+  // At least 32 dims (the fold's LDS rows): smaller heads take the general path.
+  const bool fast = a->num_tokens > 0 && p.d >= 32 && fast_path_ok(b);
+  // Fast path: one pass of the grid where it can be (16K tokens, 4 KV heads:
+  // 256 workgroups of 64 tokens), never more workgroups than CUs, since their
+  // atomics on the scales' line are served one at a time (~11 ns each).
+  const int groups = (l20kv::kScaleThreads / 64) * (fast ? 64 / (p.d / 8) : 1);
+  const int hb = std::min(p.hkv, groups);
+  const int step = l20kv::scale_rows(p.cs_dtype) * (groups / hb);  // tokens per workgroup and loop pass
+  int64_t chunk, blocks;
+  if (fast) {
+    blocks = std::min<int64_t>(256, ((int64_t)tokens + step - 1) / step);
+    chunk = (((int64_t)tokens + blocks - 1) / blocks + step - 1) / step * step;
+  } else {
+    // 16 waves of at least 4 tokens each; (K, V) x heads x chunks workgroups about the CUs
+    blocks = std::max<int64_t>(1, std::min<int64_t>(((int64_t)tokens + 63) / 64, 128 / std::min(p.hkv, 128)));
+    chunk = ((int64_t)tokens + blocks - 1) / blocks;
+  }
+  blocks = ((int64_t)tokens + chunk - 1) / chunk;
+  const dim3 grid = fast ? dim3((unsigned)blocks, (unsigned)((p.hkv + hb - 1) / hb))
+                         : dim3((unsigned)p.hkv, 2, (unsigned)blocks);
+  const bool single = fast && grid.x == 1 && grid.y == 1;
+  if (!single) {
+    hipLaunchKernelGGL(l20kv::kv_scales_init, dim3((unsigned)((p.hkv + 255) / 256)), dim3(256), 0, s, k_scales,
+                       v_scales, p.hkv);
+    const int32_t r = launched();
+    if (r != L20_PD_OK) return r;
+  }
+  if (fast) {
+    if (bf) launch_amax8<__bf16>(p, grid, k_scales, v_scales, hb, (int)chunk, per_head, single, s);
+    else launch_amax8<_Float16>(p, grid, k_scales, v_scales, hb, (int)chunk, per_head, single, s);
+  } else if (bf) {
+    hipLaunchKernelGGL((l20kv::kv_amax<__bf16>), grid, dim3(1024), 0, s, p, k_scales, v_scales, (int)chunk, per_head);
+  } else {
+    hipLaunchKernelGGL((l20kv::kv_amax<_Float16>), grid, dim3(1024), 0, s, p, k_scales, v_scales, (int)chunk, per_head);
+  }
   return launched();
 }
 

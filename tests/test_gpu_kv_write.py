@@ -244,6 +244,45 @@ def test_fp8_scales_match_oracle(per_head):
     np.testing.assert_array_equal(_np(k), _np(c["k"]))  # the scale pass leaves K untouched
 
 
+@pytest.mark.parametrize("per_head", [True, False])
+@pytest.mark.parametrize("tokens,hkv,d,rot,neox,cs,offset", [
+    (1, 4, 128, 128, True, torch.bfloat16, 0),      # one workgroup
+    (33, 1, 128, 128, True, torch.float32, 0),      # one row past the first pass
+    (127, 3, 64, 32, False, torch.float16, 0),      # lane groups left over, interleaved, partial rotary
+    (5000, 8, 128, 64, True, torch.bfloat16, 0),    # several passes per workgroup
+    (777, 5, 96, 96, True, torch.bfloat16, 0),      # 12 lanes a row
+    (65, 80, 256, 256, True, torch.bfloat16, 0),    # more heads than lane groups of a workgroup
+    (300, 4, 16, 16, True, torch.bfloat16, 0),      # head_dim below the fast path's
+    (2000, 4, 128, 128, True, torch.bfloat16, 4),   # 8-byte aligned rows: the general path
+])
+def test_fp8_scales_over_shapes(tokens, hkv, d, rot, neox, cs, offset, per_head):
+    """A maximum has no order: every split of the tokens over workgroups is exact."""
+    from oracle import kv_write_ref as kw
+    import l20_rope_kv
+
+    c = _case(tokens, 2 * hkv, hkv, d, rot, torch.bfloat16, cs, seed=tokens)
+    slots = c["slots"].clamp(min=0) if tokens == 1 else c["slots"].clone()
+    if tokens > 8:
+        slots[3] = c["pages"] * 16 + 5  # outside the cache: not stored
+        slots[5] = -1
+        c["k"][3] = c["v"][5] = 1e4     # so its values count for nothing
+    kc = torch.zeros(c["pages"], 16, hkv, d, dtype=torch.float8_e4m3fn).cuda()
+
+    def placed(x):  # rows `offset` elements past a 16-byte boundary
+        big = torch.zeros(tokens, hkv, d + offset, dtype=x.dtype, device="cuda")
+        view = big[..., offset:]
+        view.copy_(x)
+        return view
+
+    ks, vs = l20_rope_kv.l20_kv_fp8_scales(placed(c["k"]), placed(c["v"]), c["pos"].cuda(), c["cs"].cuda(), neox, kc,
+                                           kc.clone(), slots.cuda(), per_head=per_head)
+    stored = ((slots >= 0) & (slots < c["pages"] * 16)).numpy()
+    k_rot = kw.round_bf16(kw.rope(_np(c["k"]), _np(c["cs"])[c["pos"].numpy()], rot, neox))[stored]
+    want = [kw.fp8_scales(k_rot, per_head), kw.fp8_scales(_np(c["v"])[stored], per_head)]
+    for got, w in zip((ks, vs), want):
+        np.testing.assert_array_equal(got.cpu().numpy(), np.broadcast_to(w, hkv))
+
+
 def test_produced_fp8_cache_feeds_the_decode_op():
     """Producer -> consumer: decode tokens written by rope_and_cache (per-head scales from
     kv_fp8_scales) and compare the attention with the oracle over the same bytes."""
