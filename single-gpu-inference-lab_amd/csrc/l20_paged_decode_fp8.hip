@@ -53,7 +53,9 @@
 namespace l20pd {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -145,8 +147,14 @@ struct PartialParams {
 // Element helpers
 // ---------------------------------------------------------------------------
 template <typename QT> struct MfmaTypes;
-template <> struct MfmaTypes<__bf16> { typedef bf16x8 vec8; };
-template <> struct MfmaTypes<_Float16> { typedef f16x8 vec8; };
+template <> struct MfmaTypes<__bf16> {
+  typedef bf16x8 vec8;
+  typedef bf16x4 vec4;
+};
+template <> struct MfmaTypes<_Float16> {
+  typedef f16x8 vec8;
+  typedef f16x4 vec4;
+};
 
 // Eight fp8 codes (two dwords) -> eight bf16 / f16 MFMA operand elements,
 // exact (every e4m3fn and every e5m2 value is representable in both).
@@ -197,6 +205,14 @@ __device__ __forceinline__ f32x4 mfma16(const bf16x8 &a, const bf16x8 &b, f32x4 
 }
 __device__ __forceinline__ f32x4 mfma16(const f16x8 &a, const f16x8 &b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+}
+// The 16-wide k of a 16-token block: lane l holds k = 4 (l / 16) + i.
+__device__ __forceinline__ f32x4 mfma16(const bf16x4 &a, const bf16x4 &b, f32x4 c) {
+  typedef short s16x4 __attribute__((ext_vector_type(4)));
+  return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4 mfma16(const f16x4 &a, const f16x4 &b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0);
 }
 
 // Empty asm statements that take a value in VGPRs: the loads producing it
@@ -425,7 +441,15 @@ struct KvUnit {
   // Softmax probabilities: f16 for fp8 caches (V converted to f16), the
   // cache's own type for 16-bit caches.
   typedef typename std::conditional<KT != 1, _Float16, QT>::type PT;
-  typedef typename MfmaTypes<PT>::vec8 pvec8;
+  // One block's scores per lane and query tile: 8 (two 16-token MFMA tiles) or
+  // 4 (one); the PV product's k is the block: 32 or 16 tokens wide.  (A 16-token
+  // block carried as a half-empty 32-token one did twice the softmax and masked
+  // every block: hybrid tree attention, 24 drafts over 4 x 3999 bf16 tokens,
+  // 76.5 -> 75.7 us per call; one query tile waits for memory and is unchanged.)
+  static constexpr int NE = KT != 1 ? 8 : 4;
+  static constexpr int NTL = NE / 4;
+  typedef typename std::conditional<KT != 1, typename MfmaTypes<PT>::vec8, typename MfmaTypes<PT>::vec4>::type pvec;
+  typedef int pwords __attribute__((ext_vector_type(NE / 2)));
   static constexpr int kTok = KT != 1 ? 32 : 16;  // tokens per block
   // P is rounded to the MFMA operand type, 11 significant bits (f16) or 8
   // (bf16), while the softmax denominator sums it unrounded.  Equal scores
@@ -632,8 +656,7 @@ struct KvUnit {
     // beyond the unit read from page 0) and tokens of an invalid page may hold
     // arbitrary bytes, NaN codes included: zero their V so that p = 0
     // contributes exactly 0.  K needs no fix-up: their scores are replaced by
-    // -inf below.  A 16-bit block has one tile; its second-tile slots are
-    // empty (score -inf, V zero).
+    // -inf below.  A 16-bit block has one tile.
     const bool bad0 = __builtin_amdgcn_readlane(pid, KT != 1 ? 2 * blk : blk) < 0;
     const bool bad1 = KT != 1 ? __builtin_amdgcn_readlane(pid, 2 * blk + 1) < 0 : true;
     if constexpr (KT != 1) {
@@ -664,11 +687,11 @@ struct KvUnit {
     }
     if constexpr (kKLines) k_to_mfma(r, kx, (int)(threadIdx.x & 15), j);
     // ---- S^T = K . Q^T ----
-    f32x4 sc[NQT][2];
+    f32x4 sc[NQT][NTL];
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
-      sc[qt][0] = f32x4{0.f, 0.f, 0.f, 0.f};
-      sc[qt][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int T = 0; T < NTL; ++T) sc[qt][T] = f32x4{0.f, 0.f, 0.f, 0.f};
     }
     if constexpr (KT != 1) {
 #pragma unroll
@@ -692,17 +715,17 @@ struct KvUnit {
     // r.k is consumed: the refill's K loads may overwrite it
     after_scores();
     // ---- online softmax (log2 domain) ----
-    const bool need_mask = (tok0 + kTok - 1 > min_lim) || bad0 || bad1;
-    pvec8 pop[NQT];
-    pvec8 pop_lo[kSplitP ? NQT : 1];
+    const bool need_mask = (tok0 + kTok - 1 > min_lim) || bad0 || (NTL > 1 && bad1);
+    pvec pop[NQT];
+    pvec pop_lo[kSplitP ? NQT : 1];
 #pragma unroll
     for (int qt = 0; qt < NQT; ++qt) {
-      float x[8];
+      float x[NE];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[e] = sc[qt][e >> 2][e & 3] * c_log2;
+      for (int e = 0; e < NE; ++e) x[e] = sc[qt][e >> 2][e & 3] * c_log2;
       if (need_mask) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
+        for (int e = 0; e < NE; ++e) {
           const int t = tok0 + 16 * (e >> 2) + 4 * j + (e & 3);
           bool vis;
           if constexpr (TREE)
@@ -714,7 +737,7 @@ struct KvUnit {
       }
       float mloc = x[0];
 #pragma unroll
-      for (int e = 1; e < 8; ++e) mloc = fmaxf(mloc, x[e]);
+      for (int e = 1; e < NE; ++e) mloc = fmaxf(mloc, x[e]);
       mloc = wave_max_xor16_32(mloc);
       // Lazy rescale: the reference max m_run only moves when some column's
       // block max exceeds it by more than kRescaleLog2 (or it is still -inf).
@@ -731,9 +754,9 @@ struct KvUnit {
       }
       const float m_use = (m_run[qt] == -INFINITY) ? 0.0f : m_run[qt];
       float psum = 0.0f;
-      i32x4 pw, pw_lo;
+      pwords pw, pw_lo;
 #pragma unroll
-      for (int e = 0; e < 8; e += 2) {
+      for (int e = 0; e < NE; e += 2) {
         const float p0 = __builtin_amdgcn_exp2f(x[e] - m_use);
         const float p1 = __builtin_amdgcn_exp2f(x[e + 1] - m_use);
         psum += p0 + p1;
@@ -752,17 +775,17 @@ struct KvUnit {
           }
         }
       }
-      pop[qt] = __builtin_bit_cast(pvec8, pw);
-      if constexpr (kSplitP) pop_lo[qt] = __builtin_bit_cast(pvec8, pw_lo);
+      pop[qt] = __builtin_bit_cast(pvec, pw);
+      if constexpr (kSplitP) pop_lo[qt] = __builtin_bit_cast(pvec, pw_lo);
       l_run[qt] += psum;
     }
     // ---- O^T += V^T . P^T ----
     // d tile t (0 <= t < D/16) holds dims 8*(lane%16) + t (D = 128) or
     // 4*(lane%16) + t (D = 64); k slot i of the V^T and P^T operands is
-    // token 16*(i/4) + 4*(lane/16) + i%4 of the block.
+    // token 16*(i/4) + 4*(lane/16) + i%4 of the block (i < 4 in a 16-bit one).
 #pragma unroll
     for (int tp2 = 0; tp2 < NT; tp2 += 2) {
-      i32x4 wa, wb;
+      pwords wa, wb;
       if constexpr (KT != 1) {
         // d tiles tp2, tp2+1 use byte pair (c, c + 1), c = tp2 % 4, of dword tp2 / 4.
         // One byte permute interleaves tokens e and e + 1 (bytes w0.c, w1.c,
@@ -787,7 +810,7 @@ struct KvUnit {
         }
       } else {
         // d tiles tp2, tp2+1 are the low and high halves of dword tp2 / 2:
-        // pair the halves of tokens (0, 1) and (2, 3); slots 4-7 are empty
+        // pair the halves of tokens (0, 1) and (2, 3)
 #pragma unroll
         for (int e = 0; e < 4; e += 2) {
           const uint32_t w0 = (uint32_t)r.v[e][tp2 >> 1];
@@ -795,11 +818,9 @@ struct KvUnit {
           wa[e >> 1] = (int)((w0 & 0xffffu) | (w1 << 16));
           wb[e >> 1] = (int)((w0 >> 16) | (w1 & 0xffff0000u));
         }
-        wa[2] = wa[3] = 0;
-        wb[2] = wb[3] = 0;
       }
-      const pvec8 va = __builtin_bit_cast(pvec8, wa);
-      const pvec8 vb = __builtin_bit_cast(pvec8, wb);
+      const pvec va = __builtin_bit_cast(pvec, wa);
+      const pvec vb = __builtin_bit_cast(pvec, wb);
 #pragma unroll
       for (int qt = 0; qt < NQT; ++qt) {
         acc[qt][tp2] = mfma16(va, pop[qt], acc[qt][tp2]);
