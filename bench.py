@@ -339,7 +339,9 @@ def run_decode(args, mode):
     # as that kernel's split mode (then the merge): the roofline times it.
     path = cabi.launch_path(calls[0][0], lib)
     single = path == 1
-    kernel = "pd_fp8_fused" if path else "pd_fp8_partial"
+    # The other workloads' partial stage: pd_units, except with 16-bit caches (8192
+    # units at most here, past that kernel's limit for them).
+    kernel = "pd_fp8_fused" if path else "pd_units" if elem == 1 else "pd_fp8_partial"
     kernel_fn = cabi.split_out if single else cabi.partial
 
     settle_calls, settle_ms = settle(lambda i: cabi.split_out(calls[i % n_sets][0], h, lib), args.settle_ms)

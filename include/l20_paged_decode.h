@@ -209,8 +209,9 @@ int32_t l20_pd_set_spin_limit(uint32_t polls);
  * head), the splits folded in LDS, the partial_* workspace neither read nor
  * written, no merge launch --; 2 if its partial stage runs as that kernel's
  * split mode (one workgroup per (split, sequence, KV head), each writing its
- * split's partial) followed by the merge; 0 if as the persistent partial
- * kernel and the merge; -(error code) when the arguments fail
+ * split's partial) followed by the merge; 0 if as one of the two partial
+ * kernels (units spread evenly over the CUs, or the persistent work queue) and
+ * the merge; -(error code) when the arguments fail
  * l20_pd_fp8_e4m3_check.  Host only.  No reference counterpart: the reference
  * always runs its partial and reduce kernels (l20_paged_decode.cu:692-723).
  * The single launch is taken for G x q_len <= 32 (tree masks included),

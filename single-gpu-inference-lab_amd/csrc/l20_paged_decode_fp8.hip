@@ -24,6 +24,10 @@
 //    A sequence with a single split writes the final output and LSE;
 //    otherwise the fp32 partial (O / l, m, l) goes to the caller's workspace.
 //
+//  pd_units<QT, KT, D, NQT, TREE, NB>   the same per-block math with (sequence,
+//    split, KV head) units spread evenly over one workgroup per CU; the partial
+//    stage of most calls (units_fit).
+//
 //  pd_merge<QT, D, WPP, PK, SPEC>   WPP waves per (query row, q head), WPP from the split
 //    count; PK the partial element (0 fp32, 1 fp16, 2 bf16).  pd_merge_narrow<QT, D, PK>
 //    for at most eight splits and many pairs.
@@ -141,6 +145,10 @@ struct PartialParams {
   // whole sequence; otherwise the split size, one workgroup per (split,
   // sequence, KV head) writing the split's partial for the merge.
   int fused_split;
+  // pd_units only: reciprocals ceil(2^32 / d), d = the split size, the KV head
+  // count and the grid (n / d = umulhi(n, r); the host bounds n where the
+  // quotient must be exact).
+  unsigned int split_recip, heads_recip, grid_recip;
 };
 
 // ---------------------------------------------------------------------------
@@ -622,8 +630,8 @@ struct KvUnit {
     }
   }
 
-  // One block: tokens tok0 .. tok0 + kTok - 1 of the sequence, page ids in
-  // lanes kTilesPerBlock*blk (+1) of pid.  Keys at or past uEnd, on an
+  // One block: tokens tok0 .. tok0 + kTok - 1 of the sequence, bad0 (bad1) its
+  // first (second) page invalid or none.  Keys at or past uEnd, on an
   // invalid page, or hidden by the mask get score -inf and zero V.  Keys
   // before draft0 are visible to every column; key draft0 + j to draft row i
   // when j <= i (causal: lim is the lane column's last visible key) or when
@@ -647,8 +655,18 @@ struct KvUnit {
         r.k[T][c] = *reinterpret_cast<const i32x4 *>(kx + T * 16 * kKxRow + n16 * kKxRow + 16 * j + 64 * c);
   }
 
+  // The same with the page ids of the block in lanes kPagesPerBlock*blk (+1) of pid.
   template <typename F>
   __device__ __forceinline__ void compute_block(Block &r, int pid, int blk, int tok0, int uEnd, int draft0,
+                                                const int (&lim)[TREE ? 1 : NQT], int min_lim,
+                                                const int (&tree)[TREE ? NQT : 1], const qvec8 (&qop)[NQT][NS],
+                                                float c_log2, int j, char *kx, F &&after_scores) {
+    const bool bad0 = __builtin_amdgcn_readlane(pid, KT != 1 ? 2 * blk : blk) < 0;
+    const bool bad1 = KT != 1 ? __builtin_amdgcn_readlane(pid, 2 * blk + 1) < 0 : true;
+    compute_block(r, bad0, bad1, tok0, uEnd, draft0, lim, min_lim, tree, qop, c_log2, j, kx, after_scores);
+  }
+  template <typename F>
+  __device__ __forceinline__ void compute_block(Block &r, bool bad0, bool bad1, int tok0, int uEnd, int draft0,
                                                 const int (&lim)[TREE ? 1 : NQT], int min_lim,
                                                 const int (&tree)[TREE ? NQT : 1], const qvec8 (&qop)[NQT][NS],
                                                 float c_log2, int j, char *kx, F &&after_scores) {
@@ -657,8 +675,6 @@ struct KvUnit {
     // arbitrary bytes, NaN codes included: zero their V so that p = 0
     // contributes exactly 0.  K needs no fix-up: their scores are replaced by
     // -inf below.  A 16-bit block has one tile.
-    const bool bad0 = __builtin_amdgcn_readlane(pid, KT != 1 ? 2 * blk : blk) < 0;
-    const bool bad1 = KT != 1 ? __builtin_amdgcn_readlane(pid, 2 * blk + 1) < 0 : true;
     if constexpr (KT != 1) {
       if (tok0 + 32 > uEnd || bad0 || bad1) {
 #pragma unroll
@@ -1985,6 +2001,328 @@ __global__ __launch_bounds__(64 * kFusedWaves) void pd_fp8_fused(PartialParams p
   }
 }
 
+// ---------------------------------------------------------------------------
+// Partial kernel, units spread evenly over the chip
+// ---------------------------------------------------------------------------
+// A unit is one (sequence, split, KV head), numbered sequence-major, heads
+// innermost.  Every wave counts the units from the lengths (one load, a wave
+// scan); workgroup i of G, one per CU, takes the i-th of G equal runs of them.
+// Each wave takes whole units of the run (wave w units w, w + 8, ...), or, with
+// few units, P = 2, 4 or 8 waves share one, each the p-th of P parts of its
+// blocks, and their states meet in LDS.  P is the largest whose waves fill at
+// most half of the chip's (all of them with two query tiles, whose blocks take
+// twice the arithmetic): beyond that the meeting costs more than the waves give
+// (fp8, 512-token splits, us per call with P = 1, 2, 4: 8 x 4096 tokens, 8 KV
+// heads, 512 units 22.2, 19.8, 20.5; 16 x 4096, 1024 units 28.3, 29.4; 9 x 4000,
+// 4 KV heads, 288 units 21.7, 16.9, 18.9).
+//
+// Bound: HBM.  What decides is that every CU gets its share of the bytes: a CU
+// draws at most ~28 B/ns, and the persistent kernel, one workgroup per (sequence,
+// split), leaves CUs without any when a batch has fewer items than the chip has
+// CUs, and uneven ones otherwise (ragged batches, which the host cannot see).
+// And the heads of an item are read together, by neighbouring waves: a page's
+// rows hold every head, 128 bytes each, and reading them at different times costs
+// DRAM locality (equal shares cut inside units, in the same kernel otherwise:
+// 128 lognormal sequences, 4 KV heads, 45.8 -> 52 us per call; head_dim 64, 8 KV
+// heads, 90 -> 115).
+// Against the persistent kernel, us per call (512-token splits): 1 x 3000 tokens, 8
+// KV heads 31.1 -> 13.9; 8 x 4096 33.2 -> 19.8; 16 x 4096 35.7 -> 28.3; 48 x 4096
+// 76.9 -> 69.5; 128 x uniform 100-4096 108.3 -> 99.8; 32 lognormal sequences to
+// 8192, 4 KV heads, bf16 caches 63.7 -> 27.7; verification (32 x uniform to 3000,
+// 8 drafts) 51.0 -> 33.0; 128 lognormal sequences, 4 KV heads 45.7 -> 45.8; 100 x
+// 2048, 2 KV heads 25.1 -> 27.2 (the worst found).
+//
+// Block stream: NB blocks in flight across unit boundaries, as in the persistent
+// kernel.  A cursor runs NB blocks ahead of the computed block; the entries of the
+// page list for the unit after the cursor's are loaded when the cursor enters its
+// unit, and the next unit's query with them (one query tile; with two it is
+// loaded at the boundary).
+//
+// Shared units: part 0 keeps its state in registers; the others leave theirs as
+// held (f32 accumulators, maxima and lane sums) in LDS slots, and after the
+// workgroup's one barrier part 0 adds them up and writes the unit's partial (or,
+// for a sequence of one split, its rows).
+constexpr int kUnitWaves = 8;
+constexpr int kUnitHeld = 4;  // sequences per lane whose lengths stay in registers
+constexpr int kUnitMaxBatch = 64 * kUnitHeld;
+template <typename QT, int KT, int D, int NQT, bool TREE, int NB>
+__global__ __launch_bounds__(64 * kUnitWaves) void pd_units(PartialParams p) {
+  typedef KvUnit<QT, KT, D, NQT, TREE, KT != 1 && D == 128 && (NB == 1 || NQT == 1)> U;
+  typedef typename U::Block Block;
+  typedef typename U::qvec8 qvec8;
+  constexpr int kTok = U::kTok;
+  constexpr int NT = U::NT;
+  constexpr int NS = U::NS;
+  constexpr bool kQPrefetch = NQT == 1;
+  // slot w: wave w + 1 (part 0 of a unit is never the later wave)
+  __shared__ __attribute__((aligned(16))) f32x4 s_acc[kUnitWaves - 1][NQT * NT][64];
+  __shared__ float s_m[kUnitWaves - 1][NQT][64], s_l[kUnitWaves - 1][NQT][64];
+  __shared__ __attribute__((aligned(16))) char s_kx[U::kKLines ? kUnitWaves * U::kKxBytes : 16];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n16 = lane & 15;
+  const int j = lane >> 4;
+  char *const kx = s_kx + (U::kKLines ? wave * U::kKxBytes : 0);
+  const int q_len = p.q_len;
+  const int B = p.batch;
+  const int S = p.split_size;
+  const int H = p.num_kv_heads;
+  const int G = (int)gridDim.x;
+  auto n_splits = [&](int L) { return L > 0 ? (int)__umulhi((unsigned int)(L + S - 1), p.split_recip) : 1; };
+  auto unit_blocks = [&](int L, int s) { return max(1, (min(S, L - s * S) + kTok - 1) / kTok); };  // an empty one: 1
+
+  // ---- the units: lane l holds the lengths of sequences [l per, l per + per) ----
+  const int per = (B + 63) >> 6;
+  int lens[kUnitHeld], mine = 0;
+#pragma unroll
+  for (int e = 0; e < kUnitHeld; ++e) {
+    const int idx = lane * per + e;
+    lens[e] = (e < per && idx < B) ? max(0, min(p.seq_lens[idx], p.l_cap)) : -1;
+  }
+#pragma unroll
+  for (int e = 0; e < kUnitHeld; ++e)
+    if (e < per) mine += lens[e] >= 0 ? n_splits(lens[e]) : 0;
+  int incl = mine;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int t = __shfl_up(incl, off);
+    if (lane >= off) incl += t;
+  }
+  const int N = __builtin_amdgcn_readlane(incl, 63) * H;
+  constexpr int kFill = NQT == 1 ? kUnitWaves / 2 : kUnitWaves;  // waves per workgroup that sharing may fill
+  int lp = 3;  // log2 P
+  while (lp > 0 && (((int64_t)N << lp) > (int64_t)G * kFill || (S >> lp) < kTok)) --lp;
+  const int P = 1 << lp;
+  const int part = wave & (P - 1);
+  const int step_units = kUnitWaves >> lp;
+  const int unit0 = (int)__umulhi((unsigned int)N, blockIdx.x * p.grid_recip);
+  const int unit1 = (int)blockIdx.x + 1 == G ? N : (int)__umulhi((unsigned int)N, (blockIdx.x + 1) * p.grid_recip);
+  // Unit u's sequence, split, head, length and blocks.
+  auto locate = [&](int u, int &b, int &s, int &h, int &L, int &n) {
+    const int item = H == 1 ? u : (int)__umulhi((unsigned int)u, p.heads_recip);
+    h = u - item * H;
+    const int owner = __popcll(__ballot(incl <= item));
+    s = item - (__builtin_amdgcn_readlane(incl, owner) - __builtin_amdgcn_readlane(mine, owner));
+    b = owner * per;
+    L = __builtin_amdgcn_readlane(lens[0], owner);
+#pragma unroll
+    for (int e = 1; e < kUnitHeld; ++e) {
+      const int own = n_splits(L);
+      if (e < per && b == owner * per + e - 1 && s >= own) {
+        s -= own;
+        ++b;
+        L = __builtin_amdgcn_readlane(lens[e], owner);
+      }
+    }
+    n = unit_blocks(L, s);
+  };
+
+  U st;
+  st.reset();
+  qvec8 qop[NQT][NS];
+  qvec8 qopN[kQPrefetch ? NQT : 1][NS];
+  int tree[TREE ? NQT : 1] = {};
+  int treeN[TREE && kQPrefetch ? NQT : 1] = {};
+  float v_scale = 1.0f;
+  int cu = unit0 + (wave >> lp);  // the computed unit
+  const bool mine_any = cu < unit1;
+  int cb = 0, cs = 0, ch = 0, cL = 0, cN = 0;
+  if (mine_any) locate(cu, cb, cs, ch, cL, cN);
+  int ck = (cN * part) >> lp;           // the computed block of the unit
+  int cE = (cN * (part + 1)) >> lp;     // the end of the wave's part
+  bool active = ck < cE;
+
+  if (active) {
+    // Page-list entries of split s of sequence b as stored (lane t: the entry of
+    // tile t; -1 for tiles past the split or the page list), and the same as
+    // pages of the 16-token cache (-1 for an entry outside it).
+    auto load_entries = [&](int b, int s, int L) {
+      const int32_t *row = p.indptr ? p.bt + uniform_ld(p.indptr, b) : p.bt + (int64_t)b * p.bt_srow;
+      const int npages = p.indptr ? uniform_ld(p.indptr, b + 1) - uniform_ld(p.indptr, b) : p.bt_pages;
+      const int t0 = s * S / kPage;
+      const int tiles = min(npages * p.page_mult, (min(s * S + S, L) + kPage - 1) / kPage) - t0;
+      const int T = t0 + lane;
+      const int at = p.page_mult == 1 ? T : (int)__umulhi((unsigned int)T, p.page_magic);  // T / page_mult
+      int e = -1;
+      if (lane < tiles) e = row[at];
+      return e;
+    };
+    auto pages_of = [&](int e, int s) {
+      if (p.page_mult == 1) return (e >= 0 && (int64_t)e < p.num_pages) ? e : -1;
+      const int T = s * S / kPage + lane;
+      const int64_t v = (int64_t)e * p.page_mult + (T - (int)__umulhi((unsigned int)T, p.page_magic) * p.page_mult);
+      return (e >= 0 && v < p.num_pages) ? (int)v : -1;
+    };
+    // ---- the load cursor: the next block to load ----
+    int lu = cu, lb = cb, ls = cs, lh = ch, lL = cL, lk = ck, lE = cE;
+    bool lmore = true;
+    int pid = -1;                            // the cursor's unit
+    int xb = 0, xs = 0, xh = 0, xL = 0, xN = 0, entN = -1;  // the unit after it
+    int qu = -1;                             // the unit that qopN holds
+    auto prefetch_unit = [&]() {
+      if (lu + step_units >= unit1) return;
+      locate(lu + step_units, xb, xs, xh, xL, xN);
+      entN = load_entries(xb, xs, xL);
+    };
+    auto advance = [&]() {
+      if (!lmore || ++lk < lE) return;
+      lu += step_units;
+      if (lu >= unit1) {
+        lmore = false;
+        return;
+      }
+      asm volatile("" : "+v"(entN));  // the wait for the entries: here only
+      lb = xb;
+      ls = xs;
+      lh = xh;
+      lL = xL;
+      lk = 0;
+      lE = xN;
+      pid = pages_of(entN, ls);
+      prefetch_unit();
+    };
+    // ---- per unit: masks, scales ----
+    int uStart = 0, uEnd = 0, draft0 = 0, min_lim = 0;
+    int lim[TREE ? 1 : NQT] = {};
+    float c_log2 = 0.0f;
+    auto begin_unit = [&]() {
+      uStart = cs * S;
+      uEnd = min(uStart + S, cL);
+      draft0 = cL - q_len;
+      if constexpr (!TREE) {
+#pragma unroll
+        for (int qt = 0; qt < NQT; ++qt) lim[qt] = min(uEnd - 1, draft0 + (16 * qt + n16) % q_len);
+      }
+      min_lim = min(uEnd - 1, TREE ? draft0 - 1 : draft0);
+      const float k_scale = p.k_scale_ph ? uniform_ld(p.k_scale_ph, ch) : p.k_scale;
+      v_scale = p.v_scale_ph ? uniform_ld(p.v_scale_ph, ch) : p.v_scale;
+      c_log2 = k_scale * p.qk_scale_log2;
+    };
+
+    int ent = load_entries(lb, ls, lL);
+    U::load_q(p, cb, ch, qop, n16, j);
+    U::load_tree(p, cb, tree, n16);
+    if (P == 1) prefetch_unit();
+    begin_unit();
+    // Operands that later steps use on every path are pinned where they are
+    // loaded: the compiler's waits are one count per use, valid on every path
+    // into it, and a load possibly still in flight at the score product would
+    // make every block wait for all loads in flight.
+    asm volatile("" : "+v"(ent));
+    pid = pages_of(ent, ls);
+    pin_operands(qop);
+    if constexpr (TREE) pin_words(tree);
+    Block buf[NB];
+    int bad[NB];  // bit T: page T of the buffer's block is invalid or none
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+      int pg[2] = {-1, -1};
+      if (lmore) U::block_pages(pid, lk, pg);
+      U::load_pages(p, buf[i], pg, lh, 3, n16, j);
+      bad[i] = (pg[0] < 0 ? 1 : 0) | (pg[1] < 0 ? 2 : 0);
+      advance();
+    }
+    auto step = [&](Block &r, int &rbad) {
+      // the refill: the cursor's block (none: zero-extent loads, the same on every path)
+      int pg[2] = {-1, -1};
+      const int rkvh = lh;
+      if (lmore) {
+        U::block_pages(pid, lk, pg);
+        if constexpr (kQPrefetch) {
+          if (lu == cu + step_units && qu != lu) {  // the cursor has entered the next unit
+            U::load_q(p, lb, lh, qopN, n16, j);
+            U::load_tree(p, lb, treeN, n16);
+            qu = lu;
+          }
+        }
+      }
+      const bool b0 = rbad & 1, b1 = (rbad & 2) != 0;
+      constexpr bool kEarlyK = NB > 1;
+      st.compute_block(r, b0, b1, uStart + kTok * ck, uEnd, draft0, lim, min_lim, tree, qop, c_log2, j, kx, [&]() {
+        if constexpr (kEarlyK) U::load_pages(p, r, pg, rkvh, 1, n16, j);
+      });
+      U::load_pages(p, r, pg, rkvh, kEarlyK ? 2 : 3, n16, j);
+      rbad = (pg[0] < 0 ? 1 : 0) | (pg[1] < 0 ? 2 : 0);
+      advance();
+      if (NB > 1 && !active) return;  // past the end
+      if (++ck < cE) return;
+      // ---- the unit (or the wave's part of it) ends ----
+      if (P > 1) {
+        active = false;
+        return;
+      }
+      const bool one = n_splits(cL) <= 1;
+      st.template finish<true>(p, cb, ch, one, cb, cs, one && p.num_splits > 1, v_scale, n16, j, kx);
+      cu += step_units;
+      if (cu >= unit1) {
+        active = false;
+        return;
+      }
+      st.reset();
+      locate(cu, cb, cs, ch, cL, cN);
+      ck = 0;
+      cE = cN;
+      if (kQPrefetch && qu == cu) {
+        if constexpr (kQPrefetch) {
+          pin_operands(qopN);
+#pragma unroll
+          for (int s = 0; s < NS; ++s) qop[0][s] = qopN[0][s];
+          if constexpr (TREE) {
+            pin_words(treeN);
+            tree[0] = treeN[0];
+          }
+        }
+      } else {
+        U::load_q(p, cb, ch, qop, n16, j);
+        U::load_tree(p, cb, tree, n16);
+        pin_operands(qop);
+        if constexpr (TREE) pin_words(tree);
+      }
+      begin_unit();
+    };
+    // One exit, at the bottom: a path around the second step (to the loop's head,
+    // as the compiler sees a break as well) would lower the load counts that the
+    // first may leave in flight.  A step past the end computes a block of no pages,
+    // which changes nothing.
+    do {
+      step(buf[0], bad[0]);
+      if constexpr (NB > 1) step(buf[NB - 1], bad[NB - 1]);
+    } while (active);
+    if (P > 1 && part > 0) {
+#pragma unroll
+      for (int qt = 0; qt < NQT; ++qt) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) s_acc[wave - 1][qt * NT + t][lane] = st.acc[qt][t];
+        s_m[wave - 1][qt][lane] = st.m_run[qt];
+        s_l[wave - 1][qt][lane] = st.l_run[qt];
+      }
+    }
+  }
+  if (P == 1) return;
+  __syncthreads();
+  if (!mine_any || part > 0) return;
+  for (int w = 1; w < P; ++w) {
+    if ((cN * w) >> lp == (cN * (w + 1)) >> lp) continue;  // an empty part
+#pragma unroll
+    for (int qt = 0; qt < NQT; ++qt) {
+      const float m_o = s_m[wave + w - 1][qt][lane], l_o = s_l[wave + w - 1][qt][lane];
+      const float m_new = fmaxf(st.m_run[qt], m_o);
+      const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
+      const float a = __builtin_amdgcn_exp2f(st.m_run[qt] - m_use);
+      const float c = __builtin_amdgcn_exp2f(m_o - m_use);
+      st.m_run[qt] = m_new;
+      st.l_run[qt] = st.l_run[qt] * a + l_o * c;
+#pragma unroll
+      for (int t = 0; t < NT; ++t) st.acc[qt][t] = st.acc[qt][t] * a + s_acc[wave + w - 1][qt * NT + t][lane] * c;
+    }
+  }
+  if (p.v_scale_ph) v_scale = uniform_ld(p.v_scale_ph, ch);  // (an empty part 0 has not read it)
+  else v_scale = p.v_scale;
+  const bool one = n_splits(cL) <= 1;
+  st.template finish<true>(p, cb, ch, one, cb, cs, one && p.num_splits > 1, v_scale, n16, j, kx);
+}
+
 struct MergeParams {
   const void *po;
   int64_t po_srow, po_shead, po_ssplit;
@@ -2665,6 +3003,69 @@ bool fused_split_fits(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, 
   return split_mode_fills(a.split_size, triples, cus);
 }
 
+int device_cus() {
+  int dev = 0, cus = 256;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  return cus;
+}
+unsigned int recip32(int64_t d) { return d <= 1 ? 0u : (unsigned int)((((uint64_t)1 << 32) + d - 1) / d); }
+template <typename QT, int KT, int NQT, bool TREE>
+hipError_t launch_units_tiles(l20pd::PartialParams pp, int head_dim, int64_t units, hipStream_t stream) {
+  int64_t workgroups = std::min<int64_t>(units, device_cus());
+  if (const char *cap = getenv("L20_PD_MAX_WORKGROUPS")) {  // as for the persistent kernel
+    const long v = strtol(cap, nullptr, 10);
+    if (v > 0) workgroups = std::min<int64_t>(workgroups, v);
+  }
+  const dim3 grid((unsigned)workgroups), block(64 * l20pd::kUnitWaves);
+  pp.grid_recip = recip32(workgroups);
+  pp.heads_recip = recip32(pp.num_kv_heads);
+  pp.split_recip = recip32(pp.split_size);
+  // Blocks in flight per wave: two; one with two query tiles of fp8 caches (two
+  // would spill) and, as in the persistent kernel, for fp8 splits of 1024 tokens
+  // (2 x 131072 tokens, 8 KV heads 89.3 -> 87.4 us per call, 3 x 60000 69.3 -> 63.8).
+  constexpr int NB = (NQT == 1 || KT == 1) ? 2 : 1;
+  if constexpr (KT != 1 && NQT == 1)
+    if (head_dim == 128 && pp.split_size >= 1024) {
+      hipLaunchKernelGGL((l20pd::pd_units<QT, KT, 128, NQT, TREE, 1>), grid, block, 0, stream, pp);
+      return hipGetLastError();
+    }
+  if (head_dim == 128) hipLaunchKernelGGL((l20pd::pd_units<QT, KT, 128, NQT, TREE, NB>), grid, block, 0, stream, pp);
+  else hipLaunchKernelGGL((l20pd::pd_units<QT, KT, 64, NQT, TREE, NB>), grid, block, 0, stream, pp);
+  return hipGetLastError();
+}
+template <typename QT, int KT>
+hipError_t launch_units(const l20pd::PartialParams &pp, int head_dim, int nqt, int64_t units, hipStream_t stream) {
+  if (nqt == 1)
+    return pp.tree ? launch_units_tiles<QT, KT, 1, true>(pp, head_dim, units, stream)
+                   : launch_units_tiles<QT, KT, 1, false>(pp, head_dim, units, stream);
+  return pp.tree ? launch_units_tiles<QT, KT, 2, true>(pp, head_dim, units, stream)
+                 : launch_units_tiles<QT, KT, 2, false>(pp, head_dim, units, stream);
+}
+// Whether the partial stage runs as pd_units rather than the persistent kernel:
+// wherever its batch (the lengths held per wave) and the exactness of its
+// reciprocals allow, except large calls of the two kinds that measured faster on
+// the persistent kernel.  With 16-bit caches, beyond 16 units per CU at most (what
+// the host can see): 128 lognormal sequences, 4 KV heads 81.8 against 83.2 us per
+// call (8192 units at most), 64 of them 45.8 against 44.4 (4096).  At head_dim 64,
+// beyond 32: 200 x uniform to 3000, 8 KV heads 88.4 against 91.0 (9600), 100 of
+// them 53.6 against 46.5 (4800).  L20_PD_FUSED_SPLIT=0 keeps every partial stage on
+// the persistent kernel, L20_PD_UNITS=0/1 overrides the size rule (tests and
+// measurement).
+bool units_fit(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, int nqt, bool kv16) {
+  if (nqt > 2 || a.batch > l20pd::kUnitMaxBatch) return false;
+  const int64_t units = (int64_t)a.batch * a.num_kv_heads * pp.num_splits;  // at most
+  // the reciprocals' quotients are exact: tokens / split and units / heads
+  if (units >= ((int64_t)1 << 27) || units * a.num_kv_heads >= ((int64_t)1 << 32) ||
+      ((int64_t)pp.l_cap + a.split_size) * a.split_size >= ((int64_t)1 << 32))
+    return false;
+  if (const char *env = getenv("L20_PD_FUSED_SPLIT"))
+    if (env[0] == '0') return false;
+  if (const char *env = getenv("L20_PD_UNITS")) return env[0] == '1';
+  const int64_t per_cu = kv16 ? 16 : a.head_dim == 64 ? 32 : INT64_MAX / 65536;
+  return units <= per_cu * device_cus();
+}
+
 template <typename QT, int D, int WPP>
 hipError_t launch_merge_wpp(const l20pd::MergeParams &mp, int64_t pairs, hipStream_t stream) {
   constexpr int WPB = WPP > 4 ? WPP : 4;
@@ -2957,6 +3358,15 @@ int32_t run(const l20_pd_fp8_args *a, void *stream_ptr, int stages, int kinds) {
       e = bf16 ? launch_fused<__bf16, 2>(ps, D, nqt, B, H, stream) : launch_fused<_Float16, 2>(ps, D, nqt, B, H, stream);
     else
       e = bf16 ? launch_fused<__bf16, 0>(ps, D, nqt, B, H, stream) : launch_fused<_Float16, 0>(ps, D, nqt, B, H, stream);
+  } else if ((stages & kPartial) && units_fit(*a, pp, nqt, kv16)) {
+    const int D = a->head_dim;
+    const int64_t units = (int64_t)a->batch * a->num_kv_heads * pp.num_splits;
+    if (kv16)
+      e = bf16 ? launch_units<__bf16, 1>(pp, D, nqt, units, stream) : launch_units<_Float16, 1>(pp, D, nqt, units, stream);
+    else if (e5m2)
+      e = bf16 ? launch_units<__bf16, 2>(pp, D, nqt, units, stream) : launch_units<_Float16, 2>(pp, D, nqt, units, stream);
+    else
+      e = bf16 ? launch_units<__bf16, 0>(pp, D, nqt, units, stream) : launch_units<_Float16, 0>(pp, D, nqt, units, stream);
   } else if (stages & kPartial) {
     const int D = a->head_dim, B = a->batch, H = a->num_kv_heads;
     if (kv16)

@@ -316,7 +316,7 @@ def single_launch(args: L20PdFp8Args, lib: Optional[ctypes.CDLL] = None) -> bool
 def launch_path(args: L20PdFp8Args, lib: Optional[ctypes.CDLL] = None) -> int:
     """``l20_pd_single_launch``'s code: 1 the single launch (no workspace, no
     merge), 2 the single-launch kernel's split mode for the partial stage
-    (then the merge), 0 the persistent partial kernel and the merge."""
+    (then the merge), 0 a partial kernel over whole splits and the merge."""
     lib = lib or load()
     rc = lib.l20_pd_single_launch(ctypes.byref(args))
     if rc < 0:

@@ -1,0 +1,123 @@
+"""The partial kernel that spreads (sequence, split, KV head) units evenly over
+the chip (GPU), forced with L20_PD_UNITS=1: output and LSE against the oracle at
+the shapes where its schedule can go wrong -- units shared by 8, 4, 2 and 1 waves
+(fewer units than waves, parts without blocks), several units per wave (the grid
+capped), lanes holding one and several sequences, empty and one-token rows, splits
+that are not whole blocks, odd head counts, every cache type, page size and page
+list, draft rows and trees over one and two query tiles -- and the library's choice.
+"""
+
+import zlib
+
+import numpy as np
+import pytest
+import torch
+
+import pd_helpers as H
+from test_gpu_fused_split import _run
+from test_gpu_random_sweep import draw, run_case
+
+pytestmark = pytest.mark.gpu
+
+PDT = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}
+
+
+@pytest.fixture(autouse=True)
+def _units(monkeypatch):
+    monkeypatch.setenv("L20_PD_FUSED", "0")
+    monkeypatch.setenv("L20_PD_FUSED_SPLIT", "2")  # neither the split mode nor the persistent kernel
+    monkeypatch.setenv("L20_PD_UNITS", "1")
+
+
+CASES = [
+    # name, batch, hq, hkv, d, lens, q_len, per_head, fp8, page, split, pdt, workgroups (0: the CUs)
+    ("p8_one_unit", 1, 8, 1, 128, [400], 1, False, "e4m3fn", 16, 512, "fp32", 0),
+    ("p8_empty_parts", 2, 8, 2, 128, [1, 90], 1, True, "e4m3fn", 16, 512, "fp32", 0),
+    ("p2_p4", 5, 28, 4, 128, [1, 15, 1025, 2048, 600], 1, True, "e4m3fn", 16, 512, "fp16", 12),
+    ("many_per_wave", 7, 16, 2, 128, [700, 1, 0, 64, 1300, 90, 513], 1, True, "e4m3fn", 16, 64, "fp32", 1),
+    ("two_workgroups", 9, 12, 3, 128, [333, 5, 800, 64, 65, 0, 1, 1100, 127], 1, False, "e4m3fn", 16, 128, "bf16", 2),
+    ("split80", 4, 8, 2, 128, [900, 81, 80, 79], 1, False, "e4m3fn", 16, 80, "fp32", 3),
+    ("split1024", 3, 16, 2, 128, [3000, 1025, 70], 1, True, "e4m3fn", 16, 1024, "fp16", 2),
+    ("d64", 6, 14, 2, 64, [1500, 64, 0, 900, 33, 512], 1, False, "e4m3fn", 16, 256, "fp32", 2),
+    ("e5m2_pages32", 4, 16, 2, 128, [1, 1333, 2048, 64], 1, True, "e5m2", 32, 512, "fp16", 3),
+    ("pages_64", 3, 28, 4, 128, [900, 31, 2500], 1, True, "e4m3fn", 64, 256, "fp16", 2),
+    ("verify_2tiles", 5, 64, 8, 128, [1048, 17, 700, 4, 300], 4, False, "e4m3fn", 16, 256, "fp32", 2),
+    ("verify_2tiles_p", 2, 64, 8, 128, [1048, 4], 4, False, "e4m3fn", 16, 512, "fp16", 0),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
+def test_units_match_oracle(case, monkeypatch):
+    name, batch, hq, hkv, d, lens, q_len, per_head, fp8, page, split, pdt, groups = case
+    if groups:
+        monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", str(groups))
+    inp = H.make_synthetic(batch, hq, hkv, d, lens, q_len=q_len, per_head=per_head, fp8=fp8, page=page,
+                           seed=zlib.crc32(name.encode()) % 1000, garbage_tail=True)
+    out, lse, path = _run(inp, split, PDT[pdt])
+    assert path == 0
+    H.compare(out, lse, *H.run_oracle(inp))
+
+
+@pytest.mark.parametrize("batch", [65, 256])
+def test_units_many_sequences(batch, monkeypatch):
+    """Lanes hold two and four sequences' lengths."""
+    monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", "11")
+    rng = np.random.default_rng(batch)
+    lens = [int(x) for x in rng.choice([0, 1, 63, 64, 65, 200, 400], size=batch)]
+    inp = H.make_synthetic(batch, 4, 2, 64, lens, seed=batch, garbage_tail=True)
+    out, lse, _ = _run(inp, 64, torch.float32)
+    H.compare(out, lse, *H.run_oracle(inp))
+
+
+@pytest.mark.parametrize("groups", ["1", "5", "256"])
+@pytest.mark.parametrize("case", range(32))
+def test_units_random_shape(case, groups, monkeypatch):
+    monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", groups)
+    c = draw(case, seed_base=13000)
+    print(case, c, flush=True)
+    run_case(c)
+
+
+def test_units_graph_replays_match_eager():
+    inp = H.make_synthetic(6, 28, 4, 128, [900, 31, 1500, 0, 512, 77], seed=5)
+    ref, ref_lse, _ = _run(inp, 256, torch.float32)
+    q = inp["query"]
+    po, pm, ps = H.workspace(inp, 256, torch.float32)
+    out = torch.empty_like(q)
+    ks, ksph = H._scales(inp["k_scale"])
+    vs, vsph = H._scales(inp["v_scale"])
+
+    def call():
+        torch.ops.l20_stack.paged_decode_fp8_e4m3_split_out(
+            q, inp["key_cache"], inp["value_cache"], inp["block_table"], inp["seq_lens"], po, pm, ps, out, ks, vs,
+            inp["max_seq_len"], 256, inp["softmax_scale"], ksph, vsph)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        call()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        call()
+    for _ in range(3):
+        out.zero_()
+        po.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ref)
+
+
+def test_library_takes_the_units_kernel(monkeypatch):
+    """By the library's own rule (no override), bitwise the forced call's result; a batch
+    past the lengths a wave holds runs the persistent kernel, to the oracle all the same."""
+    inp = H.make_synthetic(24, 16, 2, 128, [40 + 57 * i for i in range(24)], seed=3)
+    forced, forced_lse, _ = _run(inp, 256, torch.float32)
+    for name in ("L20_PD_FUSED", "L20_PD_FUSED_SPLIT", "L20_PD_UNITS"):
+        monkeypatch.delenv(name, raising=False)
+    out, lse, path = _run(inp, 256, torch.float32)
+    assert path == 0
+    assert torch.equal(out, forced) and torch.equal(lse, forced_lse)
+    big = H.make_synthetic(257, 4, 2, 64, [1 + 7 * (i % 90) for i in range(257)], seed=4)
+    out, lse, _ = _run(big, 64, torch.float32)
+    H.compare(out, lse, *H.run_oracle(big))
