@@ -74,6 +74,12 @@ int32_t l20_pd_tree_suffix_check(const l20_pd_tree_suffix_args *args);
  * per (sequence, draft row, query head). */
 int32_t l20_pd_tree_suffix_merge(const l20_pd_tree_suffix_args *args, void *stream);
 
+/* Ancestor masks -> the bit words the decode entry points take: words[m * draft + i]
+ * bit j = mask[m][i][j] != 0, for `matrices` matrices of draft_length (1..32) rows
+ * and columns of bytes, strides in bytes (device memory; words contiguous). */
+int32_t l20_pd_tree_mask_words(const uint8_t *mask, int64_t stride_matrix, int64_t stride_row, int64_t stride_col,
+                               int32_t matrices, int32_t draft_length, int32_t *words, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

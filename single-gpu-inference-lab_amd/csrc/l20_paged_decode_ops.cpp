@@ -488,6 +488,26 @@ void tree_suffix_merge(const at::Tensor &query, const at::Tensor &suffix_key, co
   TORCH_CHECK(rc == L20_PD_OK, l20_pd_last_error());
 }
 
+// Boolean ancestor masks [..., S, S] (at most one leading dimension) as int32 bit words [..., S].
+at::Tensor tree_mask_words(const at::Tensor &mask) {
+  TORCH_CHECK(mask.is_cuda(), "ancestor_mask must be CUDA");
+  TORCH_CHECK(mask.scalar_type() == at::kBool || mask.scalar_type() == at::kByte, "ancestor_mask must be bool or uint8");
+  TORCH_CHECK((mask.dim() == 2 || mask.dim() == 3) && mask.size(-1) == mask.size(-2),
+              "ancestor_mask must be [S, S] or [B, S, S]");
+  const int64_t s = mask.size(-1);
+  TORCH_CHECK(s >= 1 && s <= 32, "tree bitmasks hold at most 32 draft tokens");
+  const int64_t matrices = mask.dim() == 3 ? mask.size(0) : 1;
+  TORCH_CHECK(matrices <= INT32_MAX, "too many ancestor masks");
+  const c10::DeviceGuard guard(mask.device());
+  at::Tensor words = at::empty(mask.sizes().slice(0, mask.dim() - 1), mask.options().dtype(at::kInt));
+  void *stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(mask.get_device()).stream();
+  const int32_t rc = l20_pd_tree_mask_words(static_cast<const uint8_t *>(mask.data_ptr()),
+                                            mask.dim() == 3 ? mask.stride(0) : 0, mask.stride(-2), mask.stride(-1),
+                                            (int32_t)matrices, (int32_t)s, words.data_ptr<int32_t>(), stream);
+  TORCH_CHECK(rc == L20_PD_OK, l20_pd_last_error());
+  return words;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(l20_stack, m) {
@@ -532,6 +552,7 @@ TORCH_LIBRARY(l20_stack, m) {
   m.def(
       "tree_suffix_merge(Tensor query, Tensor suffix_key, Tensor suffix_value, Tensor ancestor_mask, "
       "Tensor prefix_output, Tensor prefix_lse, Tensor(a!) output, float softmax_scale) -> ()");
+  m.def("tree_mask_words(Tensor mask) -> Tensor");
 }
 
 TORCH_LIBRARY_IMPL(l20_stack, CUDA, m) {
@@ -541,4 +562,5 @@ TORCH_LIBRARY_IMPL(l20_stack, CUDA, m) {
   m.impl("paged_decode_fp8_e4m3_split_out", &paged_decode_fp8_e4m3_split_out);
   m.impl("paged_decode_split_indices_out", &paged_decode_split_indices_out);
   m.impl("tree_suffix_merge", &tree_suffix_merge);
+  m.impl("tree_mask_words", &tree_mask_words);
 }

@@ -158,6 +158,25 @@ __global__ __launch_bounds__(256) void tree_suffix_merge(Params p) {
   for (int e = 0; e < E; ++e) orow[e] = (T)(acc[e] * inv);
 }
 
+// Ancestor masks as bit words: bit j of words[r] = mask row r, column j != 0.
+// Row r is row r % draft of matrix r / draft; 32 lanes take a row (draft <= 32),
+// one byte each, and a ballot forms two rows' words.  A few KB in one launch of
+// ~2 us: as tensor arithmetic it was ten launches and ~45 us of host work, most
+// of a tree-verify call (16 sequences x 8 drafts: 75 us per call).
+__global__ __launch_bounds__(256) void tree_mask_words(const uint8_t *mask, int64_t s_mat, int64_t s_row, int64_t s_col,
+                                                       int32_t *words, int64_t rows, int draft) {
+  const int lane = threadIdx.x & 63;
+  const int64_t r = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 2 + (lane >> 5);
+  const int j = lane & 31;
+  bool set = false;
+  if (r < rows && j < draft) {
+    const int64_t m = r / draft;
+    set = mask[m * s_mat + (r - m * draft) * s_row + j * s_col] != 0;
+  }
+  const uint64_t both = __ballot(set);
+  if (r < rows && j == 0) words[r] = (int32_t)(uint32_t)(lane < 32 ? both : both >> 32);
+}
+
 }  // namespace l20tv
 
 namespace {
@@ -237,6 +256,26 @@ extern "C" {
 int32_t l20_pd_tree_suffix_check(const l20_pd_tree_suffix_args *a) {
   l20pd_host::clear_error();
   return check(a);
+}
+
+int32_t l20_pd_tree_mask_words(const uint8_t *mask, int64_t stride_matrix, int64_t stride_row, int64_t stride_col,
+                               int32_t matrices, int32_t draft_length, int32_t *words, void *stream) {
+  l20pd_host::clear_error();
+  if (draft_length < 1 || draft_length > 32) return set_error(L20_PD_EINVAL, "tree bitmasks hold at most 32 draft tokens");
+  if (matrices < 0) return set_error(L20_PD_EINVAL, "matrix count must be >= 0");
+  if (matrices == 0) return L20_PD_OK;
+  if (!mask || !words) return set_error(L20_PD_EINVAL, "null tensor pointer");
+  const int64_t rows = (int64_t)matrices * draft_length;
+  hipLaunchKernelGGL(l20tv::tree_mask_words, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), mask, stride_matrix, stride_row, stride_col, words, rows,
+                     draft_length);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) {
+    char msg[256];
+    snprintf(msg, sizeof(msg), "HIP launch failed: %s", hipGetErrorString(e));
+    return set_error(L20_PD_ELAUNCH, msg);
+  }
+  return L20_PD_OK;
 }
 
 int32_t l20_pd_tree_suffix_merge(const l20_pd_tree_suffix_args *a, void *stream) {

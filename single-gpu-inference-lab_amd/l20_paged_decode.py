@@ -238,6 +238,10 @@ def _register_fake() -> None:
                                 softmax_scale):
         return None
 
+    @torch.library.register_fake("l20_stack::tree_mask_words")
+    def _tree_mask_words_fake(mask):
+        return mask.new_empty(mask.shape[:-1], dtype=torch.int32)
+
 
 load_library()
 _register_fake()

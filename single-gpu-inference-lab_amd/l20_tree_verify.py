@@ -80,6 +80,9 @@ def tree_mask_bits(ancestor_mask: torch.Tensor) -> torch.Tensor:
     s = ancestor_mask.shape[-1]
     if s > 32:
         raise ValueError("tree bitmasks hold at most 32 draft tokens")
+    if (ancestor_mask.is_cuda and s > 0 and ancestor_mask.dim() <= 3
+            and ancestor_mask.dtype in (torch.bool, torch.uint8)):
+        return torch.ops.l20_stack.tree_mask_words(ancestor_mask)  # one launch
     weights = torch.ones(s, dtype=torch.int64, device=ancestor_mask.device) << torch.arange(
         s, dtype=torch.int64, device=ancestor_mask.device)
     words = (ancestor_mask.to(torch.bool).to(torch.int64) * weights).sum(-1)

@@ -469,3 +469,21 @@ def test_contiguous_cache_tree_attention(case):
     H.compare(a, None, exp, None, check_lse=False)
     with pytest.raises(ValueError, match="cached_length"):
         tv.hybrid_tree_attention(query.cuda(), key, value, mask.cuda(), cached + 1)
+
+
+@pytest.mark.parametrize("shape", [(1, 1), (8, 8), (32, 32), (1, 3, 3), (5, 31, 31), (7, 32, 32), (300, 4, 4), (0, 4, 4)],
+                         ids=str)
+@pytest.mark.parametrize("dtype", [torch.bool, torch.uint8], ids=str)
+def test_tree_mask_words_on_the_gpu(shape, dtype):
+    """The one-launch bit words equal the tensor arithmetic's (CPU masks), transposed
+    and sliced layouts included."""
+    import l20_tree_verify as tv
+
+    g = torch.Generator().manual_seed(sum(shape))
+    host = torch.randint(0, 3, shape, generator=g).to(dtype)
+    assert torch.equal(tv.tree_mask_bits(host.cuda()).cpu(), tv.tree_mask_bits(host))
+    turned = host.cuda().transpose(-1, -2)
+    assert torch.equal(tv.tree_mask_bits(turned).cpu(), tv.tree_mask_bits(host.transpose(-1, -2)))
+    wide = torch.zeros(*shape[:-1], shape[-1] + 5, dtype=dtype, device="cuda")
+    wide[..., 3:3 + shape[-1]] = host.cuda()
+    assert torch.equal(tv.tree_mask_bits(wide[..., 3:3 + shape[-1]]).cpu(), tv.tree_mask_bits(host))
