@@ -47,11 +47,26 @@ def _num_splits(max_seq_len: int, split_size: int) -> int:
     return max(1, math.ceil(max_seq_len / split_size)) if max_seq_len > 0 else 1
 
 
+# GPU ordinal -> (gfx950, CU count).  Neither changes while the process lives, and
+# asking torch costs 2-3 us a call, a fifth of a small decode call's host time.
+_GPUS = {}
+
+
+def _gpu_facts(device) -> Tuple[bool, int]:
+    """(is a gfx950, compute units) of a GPU given as torch.device, ordinal or None (the
+    current one)."""
+    indexed = isinstance(device, torch.device) and device.type == "cuda" and device.index is not None
+    facts = _GPUS.get(device.index) if indexed else None
+    if facts is None:
+        props = torch.cuda.get_device_properties(device if device is not None else torch.cuda.current_device())
+        facts = (getattr(props, "gcnArchName", "").split(":")[0] == "gfx950", props.multi_processor_count)
+        if indexed:
+            _GPUS[device.index] = facts
+    return facts
+
+
 def is_mi355x(device: Optional[torch.device] = None) -> bool:
-    if not torch.cuda.is_available():
-        return False
-    props = torch.cuda.get_device_properties(device if device is not None else torch.cuda.current_device())
-    return getattr(props, "gcnArchName", "").split(":")[0] == "gfx950"
+    return torch.cuda.is_available() and _gpu_facts(device)[0]
 
 
 def allocate_l20_paged_split_kv_workspace(
@@ -107,12 +122,14 @@ def l20_paged_split_kv_attention_fp8(
     """
     if not is_mi355x(query.device):
         raise RuntimeError("requires an MI355X (gfx950) GPU")
-    if query.ndim != 3 or key_cache.ndim != 4 or value_cache.shape != key_cache.shape:
+    q_shape, cache_shape = query.shape, key_cache.shape
+    if len(q_shape) != 3 or len(cache_shape) != 4 or value_cache.shape != cache_shape:
         raise RuntimeError("expected Q=[B,H,D], cache=[pages,page,Hkv,D]")
-    if key_cache.dtype not in (torch.float8_e4m3fn, torch.float8_e5m2) or value_cache.dtype != key_cache.dtype:
+    cache_dtype = key_cache.dtype
+    if cache_dtype not in (torch.float8_e4m3fn, torch.float8_e5m2) or value_cache.dtype != cache_dtype:
         raise RuntimeError("key/value cache must use a torch FP8 dtype")
-    rows, num_q_heads, head_dim = query.shape
-    _, page_size, num_kv_heads, cache_dim = key_cache.shape
+    rows, num_q_heads, head_dim = q_shape
+    _, page_size, num_kv_heads, cache_dim = cache_shape
     batch = rows // q_len if q_len > 0 else -1
     if (
         head_dim not in (64, 128)
@@ -130,20 +147,20 @@ def l20_paged_split_kv_attention_fp8(
     if split_size is None:
         split_size = default_split_size(batch, num_kv_heads, max_seq_len, query.device)
     num_splits = _num_splits(max_seq_len, split_size)
-    partial_shape = (rows, num_q_heads, num_splits)
     if workspace is None:
         workspace = allocate_l20_paged_split_kv_workspace(query, max_seq_len, split_size=split_size)
     partial_output, partial_max, partial_sum, workspace_output = workspace
     if output is None:
         output = workspace_output
+    po_shape, pm_shape = partial_output.shape, partial_max.shape
     if (
-        tuple(partial_output.shape[:2]) != partial_shape[:2]
-        or partial_output.shape[2] < num_splits
-        or partial_output.shape[3] != head_dim
-        or tuple(partial_max.shape[:2]) != partial_shape[:2]
-        or partial_max.shape[2] < num_splits
-        or partial_sum.shape != partial_max.shape
-        or output.shape != query.shape
+        po_shape[:2] != (rows, num_q_heads)
+        or po_shape[2] < num_splits
+        or po_shape[3] != head_dim
+        or pm_shape[:2] != (rows, num_q_heads)
+        or pm_shape[2] < num_splits
+        or partial_sum.shape != pm_shape
+        or output.shape != q_shape
     ):
         raise RuntimeError("paged split-KV workspace shape does not match the request")
     ks, ks_ph = _split_scale(k_scale, "k_scale")
@@ -185,10 +202,11 @@ def l20_paged_split_kv_attention(
     del page_granular, grouped_gqa
     if not is_mi355x(query.device):
         raise RuntimeError("requires an MI355X (gfx950) GPU")
-    if query.ndim != 3 or key_cache.ndim != 4 or value_cache.shape != key_cache.shape:
+    q_shape, cache_shape = query.shape, key_cache.shape
+    if len(q_shape) != 3 or len(cache_shape) != 4 or value_cache.shape != cache_shape:
         raise RuntimeError("expected Q=[B,H,D], cache=[pages,page,Hkv,D]")
-    rows, num_q_heads, head_dim = query.shape
-    _, page_size, num_kv_heads, cache_dim = key_cache.shape
+    rows, num_q_heads, head_dim = q_shape
+    _, page_size, num_kv_heads, cache_dim = cache_shape
     batch = rows // q_len if q_len > 0 else -1
     if (
         head_dim not in (64, 128)
@@ -213,14 +231,15 @@ def l20_paged_split_kv_attention(
     partial_output, partial_max, partial_sum, workspace_output = workspace
     if output is None:
         output = workspace_output
+    po_shape, pm_shape = partial_output.shape, partial_max.shape
     if (
-        tuple(partial_output.shape[:2]) != (rows, num_q_heads)
-        or partial_output.shape[2] < num_splits
-        or partial_output.shape[3] != head_dim
-        or tuple(partial_max.shape[:2]) != (rows, num_q_heads)
-        or partial_max.shape[2] < num_splits
-        or partial_sum.shape != partial_max.shape
-        or output.shape != query.shape
+        po_shape[:2] != (rows, num_q_heads)
+        or po_shape[2] < num_splits
+        or po_shape[3] != head_dim
+        or pm_shape[:2] != (rows, num_q_heads)
+        or pm_shape[2] < num_splits
+        or partial_sum.shape != pm_shape
+        or output.shape != q_shape
     ):
         raise RuntimeError("paged split-KV workspace shape does not match the request")
     return torch.ops.l20_stack.paged_decode_split_out(
@@ -237,7 +256,7 @@ def default_split_size(batch: int, num_kv_heads: int, max_seq_len: int,
 
     cus = 256
     if torch.cuda.is_available():
-        cus = torch.cuda.get_device_properties(device if device is not None else 0).multi_processor_count
+        cus = _gpu_facts(device if device is not None else 0)[1]
     return int(l20_pd_cabi.load().l20_pd_default_split_size(batch, num_kv_heads, max_seq_len, cus))
 
 

@@ -42,21 +42,22 @@ def l20_rope_and_cache(
     """RoPE on Q (optional) and K in place; K/V written to the paged caches."""
     if not is_mi355x(key.device):
         raise RuntimeError("l20_rope_and_cache requires an MI355X (gfx950) GPU")
-    if key.dtype not in (torch.float16, torch.bfloat16):
+    dtype, shape, cache_dtype, cache_shape = key.dtype, key.shape, key_cache.dtype, key_cache.shape
+    if dtype not in (torch.float16, torch.bfloat16):
         raise RuntimeError("l20_rope_and_cache supports FP16 and BF16")
-    if value.dtype != key.dtype or (query is not None and query.dtype != key.dtype):
+    if value.dtype != dtype or (query is not None and query.dtype != dtype):
         raise RuntimeError("Q, K, and V must use the same dtype")
-    if key_cache.dtype not in (torch.float8_e4m3fn, key.dtype) or value_cache.dtype != key_cache.dtype:
+    if cache_dtype not in (torch.float8_e4m3fn, dtype) or value_cache.dtype != cache_dtype:
         raise RuntimeError("K/V cache must be torch.float8_e4m3fn or the model dtype")
-    if key.ndim != 3 or value.ndim != 3 or (query is not None and query.ndim != 3):
+    if len(shape) != 3 or value.ndim != 3 or (query is not None and query.ndim != 3):
         raise RuntimeError("Q, K, and V must be [tokens, heads, head_dim]")
-    if key.shape != value.shape or (query is not None and query.shape[0] != key.shape[0]):
+    if shape != value.shape or (query is not None and query.shape[0] != shape[0]):
         raise RuntimeError("Q, K, and V shapes are incompatible")
-    if key_cache.ndim != 4 or value_cache.shape != key_cache.shape:
+    if len(cache_shape) != 4 or value_cache.shape != cache_shape:
         raise RuntimeError("cache must use NHD [blocks, block, heads, dim]")
-    if key_cache.shape[2:] != key.shape[1:]:
+    if cache_shape[2:] != shape[1:]:
         raise RuntimeError("cache head shape must match K/V")
-    if positions.numel() != key.shape[0] or slot_mapping.numel() != key.shape[0]:
+    if positions.numel() != shape[0] or slot_mapping.numel() != shape[0]:
         raise RuntimeError("positions and slot_mapping must match token count")
     torch.ops.l20_stack.rope_and_cache(query, key, value, positions, cos_sin_cache, bool(is_neox), key_cache,
                                        value_cache, slot_mapping, float(k_scale), float(v_scale),
