@@ -1,10 +1,11 @@
 // Paged KV-cache producer for MI355X (gfx950): rotary embedding of Q and K
 // and the paged write of K and V into fp8 (OCP e4m3fn) or 16-bit caches.
 //
-//  kv_rope_write8<T, CT, CS>   the fast path: every Q and K head row of the
+//  kv_rope_write8<T, CT, CS, ROWS>   the fast path: every Q and K head row of the
 //    call is one row of the work; a lane owns eight contiguous dims (16-byte
-//    loads and stores), D/8 lanes a row, and each lane takes two rows with
-//    all their loads issued before any arithmetic.  A neox pair partner lies
+//    loads and stores), D/8 lanes a row, and each lane takes ROWS rows (one in
+//    small calls, else two) with all their loads issued before any arithmetic;
+//    row numbers are 32-bit (the 64-bit divisions cost a small call ~0.1 us).  A neox pair partner lies
 //    half/8 lanes away in the same row and is exchanged with a lane shuffle;
 //    cos and sin arrive as 8 (neox) or 4 (interleaved) consecutive values.
 //    Taken when rows, caches and the cos/sin table are 16-byte aligned,
@@ -262,13 +263,11 @@ __device__ __forceinline__ int quant4(const float (&x)[4], float scale) {
   return w;
 }
 
-constexpr int kRowsPerLane = 2;
-
 // Rows [0, rows_q) are Q head rows (token r / Hq, head r % Hq), the next
 // rows_k are K head rows (token r / Hkv): rotated in place, and for K also the
 // K and V cache writes.  Four waves; a lane group of lpr = D/8 lanes per row.
-template <typename T, int CT, int CS>
-__global__ __launch_bounds__(256) void kv_rope_write8(Params p, int64_t rows_q, int64_t rows_all) {
+template <typename T, int CT, int CS, int ROWS>
+__global__ __launch_bounds__(256) void kv_rope_write8(Params p, uint32_t rows_q, uint32_t rows_all) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
@@ -279,31 +278,33 @@ __global__ __launch_bounds__(256) void kv_rope_write8(Params p, int64_t rows_q, 
   const int e0 = 8 * l;
   const int half = p.rot >> 1;
   const bool rot_lane = e0 < p.rot;
-  const int64_t first = (int64_t)blockIdx.x * (4 * rpw * kRowsPerLane);
+  const uint32_t first = blockIdx.x * (uint32_t)(4 * rpw * ROWS);
 
   // ---- loads of all of this lane's rows ----
-  i32x4 xw[kRowsPerLane], vw[kRowsPerLane];
-  int64_t pos[kRowsPerLane], slot[kRowsPerLane];
-  float ksc[kRowsPerLane], vsc[kRowsPerLane];  // the K row's cache scales (loaded with the row)
-  T *row[kRowsPerLane];
-  int head[kRowsPerLane];
-  bool live[kRowsPerLane], is_k[kRowsPerLane];
+  i32x4 xw[ROWS], vw[ROWS];
+  int64_t pos[ROWS], slot[ROWS];
+  float ksc[ROWS], vsc[ROWS];  // the K row's cache scales (loaded with the row)
+  T *row[ROWS];
+  int head[ROWS];
+  bool live[ROWS], is_k[ROWS];
 #pragma unroll
-  for (int u = 0; u < kRowsPerLane; ++u) {
-    const int64_t r = first + (int64_t)(u * 4 + wave) * rpw + g;
+  for (int u = 0; u < ROWS; ++u) {
+    const uint32_t r = first + (uint32_t)((u * 4 + wave) * rpw + g);
     live[u] = g < rpw && r < rows_all;
     is_k[u] = r >= rows_q;
     int64_t t = 0;
     int h = 0;
     if (live[u]) {
       if (!is_k[u]) {
-        t = r / p.hq;
-        h = (int)(r - t * p.hq);
+        const uint32_t q = r / (uint32_t)p.hq;
+        t = q;
+        h = (int)(r - q * (uint32_t)p.hq);
         row[u] = reinterpret_cast<T *>(p.q) + t * p.q_st + (int64_t)h * p.q_sh;
       } else {
-        const int64_t rk = r - rows_q;
-        t = rk / p.hkv;
-        h = (int)(rk - t * p.hkv);
+        const uint32_t rk = r - rows_q;
+        const uint32_t q = rk / (uint32_t)p.hkv;
+        t = q;
+        h = (int)(rk - q * (uint32_t)p.hkv);
         row[u] = reinterpret_cast<T *>(p.k) + t * p.k_st + (int64_t)h * p.k_sh;
         vw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(reinterpret_cast<const T *>(p.v) + t * p.v_st +
                                                  (int64_t)h * p.v_sh + e0));
@@ -319,14 +320,14 @@ __global__ __launch_bounds__(256) void kv_rope_write8(Params p, int64_t rows_q, 
     head[u] = h;
   }
   // ---- cos / sin of the lanes' dims ----
-  CosSin<CS> cs[kRowsPerLane];
+  CosSin<CS> cs[ROWS];
 #pragma unroll
-  for (int u = 0; u < kRowsPerLane; ++u) {
+  for (int u = 0; u < ROWS; ++u) {
     if (live[u] && rot_lane) load_row_cs<CS>(p, pos[u], e0, half, cs[u]);
   }
   // ---- rotate, store back, write the caches ----
 #pragma unroll
-  for (int u = 0; u < kRowsPerLane; ++u) {
+  for (int u = 0; u < ROWS; ++u) {
     // the neox partner's words, from the lane half/8 away in the same row (every lane shuffles)
     const int src = g * lpr + (e0 < half ? l + (half >> 3) : l - (half >> 3));
     i32x4 pw;
@@ -702,17 +703,28 @@ bool fast_path_ok(const l20_pd_kv_write_args &a) {
   return true;
 }
 
-template <typename T, int CT>
-void launch_fast(const l20kv::Params &p, int cs_dtype, int64_t rows_q, int64_t rows_all, hipStream_t s) {
-  const int lpr = p.d / 8;
-  const int64_t rows_per_wg = (int64_t)4 * (64 / lpr) * l20kv::kRowsPerLane;
+template <typename T, int CT, int ROWS>
+void launch_fast_rows(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uint32_t rows_all, hipStream_t s) {
+  const int64_t rows_per_wg = (int64_t)4 * (64 / (p.d / 8)) * ROWS;
   const dim3 grid((unsigned)((rows_all + rows_per_wg - 1) / rows_per_wg));
   if (cs_dtype == 2)
-    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 2>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 2, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
   else if (cs_dtype == 1)
-    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 1>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 1, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
   else
-    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+}
+
+// One row per lane while the workgroups of one fit the chip at once (8 per CU: a
+// small call is one chain of dependent loads, and a second row only lengthens
+// it), else two.  32 heads of 128, fp8 cache, us per call with one and two, in a
+// graph: 16 tokens 3.44, 4.30; 128 tokens 4.01, 4.89; 1024 (2048 workgroups of
+// one) 6.21, 6.61; 1500 8.81, 8.30; 16384 64.8, 64.2.
+template <typename T, int CT>
+void launch_fast(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uint32_t rows_all, hipStream_t s) {
+  const int64_t one = ((int64_t)rows_all + 4 * (64 / (p.d / 8)) - 1) / (4 * (64 / (p.d / 8)));
+  if (one <= 2048) launch_fast_rows<T, CT, 1>(p, cs_dtype, rows_q, rows_all, s);
+  else launch_fast_rows<T, CT, 2>(p, cs_dtype, rows_q, rows_all, s);
 }
 
 template <typename T>
@@ -753,9 +765,10 @@ int32_t l20_pd_rope_and_cache(const l20_pd_kv_write_args *a, void *stream) {
   const l20kv::Params p = params(*a);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const bool bf = a->dtype == L20_PD_BF16;
-  if (fast_path_ok(*a)) {
-    const int64_t rows_q = (int64_t)a->num_tokens * p.hq;
-    const int64_t rows_all = rows_q + (int64_t)a->num_tokens * p.hkv;
+  // (row numbers in 32 bits, with room for the last workgroup's)
+  if (fast_path_ok(*a) && (int64_t)a->num_tokens * ((int64_t)p.hq + p.hkv) < ((int64_t)1 << 31)) {
+    const uint32_t rows_q = (uint32_t)((int64_t)a->num_tokens * p.hq);
+    const uint32_t rows_all = (uint32_t)((int64_t)a->num_tokens * ((int64_t)p.hq + p.hkv));
     const bool fp8 = a->cache_dtype == L20_PD_KV_FP8_E4M3;
     if (bf) {
       if (fp8) launch_fast<__bf16, 0>(p, p.cs_dtype, rows_q, rows_all, s);
