@@ -74,6 +74,14 @@ int32_t l20_pd_tree_suffix_check(const l20_pd_tree_suffix_args *args);
  * per (sequence, draft row, query head). */
 int32_t l20_pd_tree_suffix_merge(const l20_pd_tree_suffix_args *args, void *stream);
 
+/* The prefix pass's page table, lengths and ancestor words of hybrid tree attention:
+ * table[e][t] (int32 [entries, width], or NULL: left as it is) = pages of sequence
+ * e / chunks: pages[b * stride_row + t * stride_col], or with is_base
+ * pages[b * stride_row] + t; lens[e] = length; words[0 .. cols) = all `cols` bits set. */
+int32_t l20_pd_tree_prefix_setup(const int32_t *pages, int64_t stride_row, int64_t stride_col, int32_t is_base,
+                                 int32_t *table, int32_t width, int32_t entries, int32_t chunks, int32_t length,
+                                 int32_t cols, int32_t *lens, int32_t *words, void *stream);
+
 /* Ancestor masks -> the bit words the decode entry points take: words[m * draft + i]
  * bit j = mask[m][i][j] != 0, for `matrices` matrices of draft_length (1..32) rows
  * and columns of bytes, strides in bytes (device memory; words contiguous). */

@@ -488,6 +488,36 @@ void tree_suffix_merge(const at::Tensor &query, const at::Tensor &suffix_key, co
   TORCH_CHECK(rc == L20_PD_OK, l20_pd_last_error());
 }
 
+// The page table, lengths and ancestor words of hybrid tree attention's prefix pass.
+void tree_prefix_setup(const at::Tensor &pages, bool is_base, int64_t chunks, int64_t length, int64_t cols,
+                       const std::optional<at::Tensor> &table, const at::Tensor &lens, const at::Tensor &words) {
+  TORCH_CHECK(lens.is_cuda() && lens.scalar_type() == at::kInt && lens.dim() == 1 && lens.is_contiguous(),
+              "lens must be contiguous int32 [entries]");
+  TORCH_CHECK(words.scalar_type() == at::kInt && words.dim() == 1 && words.is_contiguous() && words.size(0) == cols,
+              "words must be contiguous int32 [cols]");
+  TORCH_CHECK(pages.scalar_type() == at::kInt && pages.dim() == (is_base ? 1 : 2),
+              "pages must be an int32 block table or page base");
+  const int64_t entries = lens.size(0);
+  TORCH_CHECK(chunks >= 1 && pages.size(0) * chunks == entries, "pages must have entries / chunks rows");
+  for (const at::Tensor *t : {&pages, &words}) check_same_device(*t, lens, "every tensor");
+  const bool has = table.has_value() && table->defined();
+  if (has) {
+    TORCH_CHECK(table->scalar_type() == at::kInt && table->dim() == 2 && table->is_contiguous() &&
+                    table->size(0) == entries && (is_base || table->size(1) <= pages.size(1)),
+                "table must be contiguous int32 [entries, pages]");
+    TORCH_CHECK(table->size(1) <= INT32_MAX, "too many pages");
+    check_same_device(*table, lens, "table");
+  }
+  TORCH_CHECK(entries <= 65535 && chunks <= INT32_MAX && length >= 0 && length <= INT32_MAX, "too many entries");
+  const c10::DeviceGuard guard(lens.device());
+  void *stream = at::hip::getCurrentHIPStreamMasqueradingAsCUDA(lens.get_device()).stream();
+  const int32_t rc = l20_pd_tree_prefix_setup(
+      pages.data_ptr<int32_t>(), pages.stride(0), is_base ? 0 : pages.stride(1), is_base ? 1 : 0,
+      has ? table->data_ptr<int32_t>() : nullptr, has ? (int32_t)table->size(1) : 0, (int32_t)entries, (int32_t)chunks,
+      (int32_t)length, (int32_t)cols, lens.data_ptr<int32_t>(), words.data_ptr<int32_t>(), stream);
+  TORCH_CHECK(rc == L20_PD_OK, l20_pd_last_error());
+}
+
 // Boolean ancestor masks [..., S, S] (at most one leading dimension) as int32 bit words [..., S].
 at::Tensor tree_mask_words(const at::Tensor &mask) {
   TORCH_CHECK(mask.is_cuda(), "ancestor_mask must be CUDA");
@@ -553,6 +583,9 @@ TORCH_LIBRARY(l20_stack, m) {
       "tree_suffix_merge(Tensor query, Tensor suffix_key, Tensor suffix_value, Tensor ancestor_mask, "
       "Tensor prefix_output, Tensor prefix_lse, Tensor(a!) output, float softmax_scale) -> ()");
   m.def("tree_mask_words(Tensor mask) -> Tensor");
+  m.def(
+      "tree_prefix_setup(Tensor pages, bool is_base, int chunks, int length, int cols, Tensor(a!)? table, "
+      "Tensor(b!) lens, Tensor(c!) words) -> ()");
 }
 
 TORCH_LIBRARY_IMPL(l20_stack, CUDA, m) {
@@ -563,4 +596,5 @@ TORCH_LIBRARY_IMPL(l20_stack, CUDA, m) {
   m.impl("paged_decode_split_indices_out", &paged_decode_split_indices_out);
   m.impl("tree_suffix_merge", &tree_suffix_merge);
   m.impl("tree_mask_words", &tree_mask_words);
+  m.impl("tree_prefix_setup", &tree_prefix_setup);
 }

@@ -242,6 +242,10 @@ def _register_fake() -> None:
     def _tree_mask_words_fake(mask):
         return mask.new_empty(mask.shape[:-1], dtype=torch.int32)
 
+    @torch.library.register_fake("l20_stack::tree_prefix_setup")
+    def _tree_prefix_setup_fake(pages, is_base, chunks, length, cols, table, lens, words):
+        return None
+
 
 load_library()
 _register_fake()

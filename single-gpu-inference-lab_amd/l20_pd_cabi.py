@@ -47,6 +47,7 @@ EXPORTED = (
     "l20_pd_tree_suffix_check",
     "l20_pd_tree_suffix_merge",
     "l20_pd_tree_mask_words",
+    "l20_pd_tree_prefix_setup",
 )
 
 _i32, _i64, _f32, _vp = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_void_p

@@ -368,20 +368,29 @@ def hybrid_tree_attention_paged_prefix(
         if padded != draft:
             qb[:, draft:].zero_()
         rows_q = qb.view(entries * cols, num_q_heads, head_dim)
-    pages = max(1, math.ceil(cached_length / page))
-    if contiguous_pages:
-        ramp = ws.constant("ramp", lambda: torch.arange(pages, dtype=torch.int32, device=dev), (pages,), dev)
-        table = ws.buffer("table", (entries, pages), torch.int32, dev)
-        torch.add(page_base.to(torch.int32)[:, None, None], ramp[None, None, :], out=table.view(batch, chunks, pages))
-    elif chunks > 1:
-        table = ws.buffer("table", (entries, block_table.shape[1]), torch.int32, dev)
-        table.view(batch, chunks, -1).copy_(block_table[:, None, :].expand(batch, chunks, block_table.shape[1]))
-    else:
-        table = block_table
     lens = ws.buffer("lens", (entries,), torch.int32, dev)
-    lens.fill_(int(cached_length))
     words = ws.buffer("words", (cols,), torch.int32, dev)
-    words.fill_(-1 if cols == 32 else (1 << cols) - 1)
+    if contiguous_pages:
+        pages = max(1, math.ceil(cached_length / page))
+        source = page_base.to(torch.int32)
+        table = ws.buffer("table", (entries, pages), torch.int32, dev)
+        filled = table
+    elif chunks > 1:
+        source = block_table.to(torch.int32)
+        table = filled = ws.buffer("table", (entries, block_table.shape[1]), torch.int32, dev)
+    else:
+        source = table = block_table
+        filled = None  # used as it is
+    if source.dtype == torch.int32 and source.device == lens.device and 0 < entries <= 65535:
+        torch.ops.l20_stack.tree_prefix_setup(source, contiguous_pages, chunks, int(cached_length), cols, filled, lens,
+                                              words)
+    else:  # the decode op reports what does not fit
+        lens.fill_(int(cached_length))
+        words.fill_(-1 if cols == 32 else (1 << cols) - 1)
+        if filled is not None:
+            filled.view(batch, chunks, -1).copy_(
+                source[:, None, None] + torch.arange(filled.shape[1], dtype=torch.int32, device=source.device)
+                if contiguous_pages else source[:, None, :].expand(batch, chunks, filled.shape[1]))
     if split_size is None:
         split_size = default_split_size(entries, num_kv_heads, int(cached_length), dev)
     n_s = max(1, math.ceil(cached_length / split_size)) if cached_length > 0 else 1

@@ -487,3 +487,29 @@ def test_tree_mask_words_on_the_gpu(shape, dtype):
     wide = torch.zeros(*shape[:-1], shape[-1] + 5, dtype=dtype, device="cuda")
     wide[..., 3:3 + shape[-1]] = host.cuda()
     assert torch.equal(tv.tree_mask_bits(wide[..., 3:3 + shape[-1]]).cpu(), tv.tree_mask_bits(host))
+
+
+@pytest.mark.parametrize("batch,chunks,width,cols", [(1, 1, 1, 1), (3, 2, 257, 32), (2, 3, 256, 31), (5, 4, 13, 8)])
+@pytest.mark.parametrize("source", ["rows", "strided", "base", "kept"])
+def test_tree_prefix_setup(batch, chunks, width, cols, source):
+    """Page table (from rows, strided rows or page bases, or left alone), lengths and words."""
+    entries = batch * chunks
+    g = torch.Generator().manual_seed(width)
+    rows = torch.randint(0, 1000, (batch, width), generator=g, dtype=torch.int32).cuda()
+    pages = rows
+    if source == "strided":
+        wide = torch.zeros(batch, 2 * width + 3, dtype=torch.int32, device="cuda")
+        pages = wide[:, 1:1 + 2 * width:2]
+        pages.copy_(rows)
+    elif source == "base":
+        pages = rows[:, 0].contiguous()
+        rows = pages[:, None] + torch.arange(width, dtype=torch.int32, device="cuda")
+    table = torch.full((entries, width), -7, dtype=torch.int32, device="cuda")
+    lens = torch.zeros(entries, dtype=torch.int32, device="cuda")
+    words = torch.zeros(cols, dtype=torch.int32, device="cuda")
+    torch.ops.l20_stack.tree_prefix_setup(pages, source == "base", chunks, 1234, cols,
+                                          None if source == "kept" else table, lens, words)
+    want = table if source == "kept" else rows.repeat_interleave(chunks, 0)
+    assert torch.equal(table, want)
+    assert bool((lens == 1234).all())
+    assert bool((words == (-1 if cols == 32 else (1 << cols) - 1)).all())
