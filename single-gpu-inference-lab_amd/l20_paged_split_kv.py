@@ -249,15 +249,17 @@ def l20_paged_split_kv_attention(
     )
 
 
+def gpu_cus(device: Optional[torch.device] = None) -> int:
+    """Compute units of the device (GPU 0 by default; 256, an MI355X, without a GPU)."""
+    return _gpu_facts(device if device is not None else 0)[1] if torch.cuda.is_available() else 256
+
+
 def default_split_size(batch: int, num_kv_heads: int, max_seq_len: int,
                        device: Optional[torch.device] = None) -> int:
     """Split size from the library's heuristic for the device's CU count."""
     import l20_pd_cabi
 
-    cus = 256
-    if torch.cuda.is_available():
-        cus = _gpu_facts(device if device is not None else 0)[1]
-    return int(l20_pd_cabi.load().l20_pd_default_split_size(batch, num_kv_heads, max_seq_len, cus))
+    return int(l20_pd_cabi.load().l20_pd_default_split_size(batch, num_kv_heads, max_seq_len, gpu_cus(device)))
 
 
 def should_use_l20_paged_split_kv(batch: int, max_seq_len: int) -> bool:

@@ -42,7 +42,7 @@ from typing import Optional, Tuple, Union
 import torch
 
 import l20_paged_decode  # noqa: F401  (loads the TORCH_LIBRARY extension)
-from l20_paged_split_kv import default_split_size, is_mi355x
+from l20_paged_split_kv import default_split_size, gpu_cus, is_mi355x
 
 Scale = Union[float, torch.Tensor]
 MAX_COLUMNS = 32  # query columns (draft rows x GQA group) of one kernel work item
@@ -91,6 +91,26 @@ def tree_mask_bits(ancestor_mask: torch.Tensor) -> torch.Tensor:
     return words.to(torch.int32)
 
 
+def _tree_split_size(entries: int, num_kv_heads: int, columns: int, max_len: int, device) -> int:
+    """Split size of a tree call whose caller names none: the library's, except that
+    calls of more than 16 query columns take at least 512 tokens once that leaves more
+    units (entry, split, KV head) than the GPU has CUs, and 1024 once that leaves four
+    times as many.  Every such unit writes 32 fp32 rows (16 KB at head_dim 128), which
+    at the library's 128 or 256 tokens cost more than the finer splits give (us per
+    call at 128, 256, 512, 1024 tokens; 32 / 8 heads, 8 drafts: 16 x 500-3000 tokens
+    37.0, 34.9, 33.8, 35.9; 64 x 500-2000 83.6, 68.3, 56.9, 54.5; 24 drafts beside 4 x
+    3999 bf16 tokens 84.8, 66.3, 61.1, 64.7; with 8 columns, 16 x 500-3000 20.5, 18.9,
+    19.9, 25.0)."""
+    split = default_split_size(entries, num_kv_heads, max_len, device)
+    if columns > 16:
+        cus = gpu_cus(device)
+        for wider, fill in ((512, 1), (1024, 4)):
+            units = entries * num_kv_heads * math.ceil(max_len / wider)
+            if split < wider and (units >= fill * cus if fill > 1 else units > cus):
+                split = wider
+    return split
+
+
 def _scale_args(scale: Scale) -> Tuple[float, Optional[torch.Tensor]]:
     if isinstance(scale, torch.Tensor):
         if scale.numel() == 1:
@@ -109,7 +129,8 @@ def _paged_call(rows_q: torch.Tensor, key_cache: torch.Tensor, value_cache: torc
     batch = rows_q.shape[0] // q_len
     num_q_heads, head_dim = rows_q.shape[1], rows_q.shape[2]
     if split_size is None:
-        split_size = default_split_size(batch, key_cache.shape[2], max_seq_len, rows_q.device)
+        split_size = _tree_split_size(batch, key_cache.shape[2], q_len * (num_q_heads // key_cache.shape[2]),
+                                      max_seq_len, rows_q.device)
     if partials is None:
         n_s = max(1, math.ceil(max_seq_len / split_size)) if max_seq_len > 0 else 1
         shape = (rows_q.shape[0], num_q_heads, n_s)
@@ -392,7 +413,7 @@ def hybrid_tree_attention_paged_prefix(
                 source[:, None, None] + torch.arange(filled.shape[1], dtype=torch.int32, device=source.device)
                 if contiguous_pages else source[:, None, :].expand(batch, chunks, filled.shape[1]))
     if split_size is None:
-        split_size = default_split_size(entries, num_kv_heads, int(cached_length), dev)
+        split_size = _tree_split_size(entries, num_kv_heads, cols * group, int(cached_length), dev)
     n_s = max(1, math.ceil(cached_length / split_size)) if cached_length > 0 else 1
     n_rows = entries * cols
     partials = (ws.buffer("partial_output", (n_rows, num_q_heads, n_s, head_dim), torch.float32, dev),

@@ -76,3 +76,17 @@ def test_reference_policy_helpers():
     assert [tv.l20_tree_attention_block_t(n) for n in (0, 4095, 4096, 100000)] == [64, 64, 128, 128]
     for n in (0, 4095, 4096):
         tv._check_block_t(tv.l20_tree_attention_block_t(n))  # accepted by the entry points
+
+
+@pytest.mark.parametrize("entries,heads,columns,length,split", [
+    (16, 8, 32, 3000, 512),    # 768 units of 512 tokens, 384 of 1024
+    (64, 8, 32, 2000, 1024),   # 1024 units of 1024
+    (63, 8, 32, 2000, 512),    # 1008: one sequence short of it
+    (16, 8, 16, 3000, None),   # one query tile: the library's
+    (4, 8, 32, 512, None),     # 32 units of 512: the library's
+    (1, 8, 32, 40000, 1024),   # the library's own 1024 stays
+])
+def test_tree_split_size_rule(entries, heads, columns, length, split):
+    """256 CUs (no GPU here, or an MI355X)."""
+    want = tv.default_split_size(entries, heads, length) if split is None else split
+    assert tv._tree_split_size(entries, heads, columns, length, None) == want
