@@ -2016,10 +2016,11 @@ __global__ __launch_bounds__(64 * kFusedWaves) void pd_fp8_fused(PartialParams p
 // heads, 512 units 22.2, 19.8, 20.5; 16 x 4096, 1024 units 28.3, 29.4; 9 x 4000,
 // 4 KV heads, 288 units 21.7, 16.9, 18.9).
 //
-// Bound: HBM.  What decides is that every CU gets its share of the bytes: a CU
-// draws at most ~28 B/ns, and the persistent kernel, one workgroup per (sequence,
-// split), leaves CUs without any when a batch has fewer items than the chip has
-// CUs, and uneven ones otherwise (ragged batches, which the host cannot see).
+// Bound: HBM.  What decides is that every CU gets its share of the bytes: with the
+// 128 KB that eight waves of two blocks keep in flight a CU draws ~28 B/ns, and the
+// persistent kernel, one workgroup per (sequence, split), leaves CUs without any
+// when a batch has fewer items than the chip has CUs, and uneven ones otherwise
+// (ragged batches, which the host cannot see).
 // And the heads of an item are read together, by neighbouring waves: a page's
 // rows hold every head, 128 bytes each, and reading them at different times costs
 // DRAM locality (equal shares cut inside units, in the same kernel otherwise:
