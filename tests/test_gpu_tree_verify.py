@@ -325,6 +325,33 @@ def test_tree_suffix_merge_c_abi_against_closed_form(d, qdt, prefix_f32):
     assert np.all(np.abs(got - exp) <= rel * np.abs(exp) + 1e-3)
 
 
+@pytest.mark.parametrize("b,s,hq,hkv,d", [(1, 1, 1, 1, 128), (3, 8, 7, 1, 64), (2, 9, 6, 2, 128), (1, 64, 3, 3, 64)])
+def test_tree_suffix_merge_reads_nothing_it_may_not_use(b, s, hq, hkv, d):
+    """Row counts that leave waves over (rows % 4 != 0), 1, 8, 9 and 64 drafts (around the
+    batch of eight), NaN in a draft no row sees and in the output of an empty prefix."""
+    import l20_pd_cabi as cabi
+
+    g = torch.Generator().manual_seed(s)
+    q, po = (torch.randn(b, s, hq, d, generator=g).half() for _ in range(2))
+    sk, sv = (torch.randn(b, s, hkv, d, generator=g).half() for _ in range(2))
+    mask = torch.ones(s, s, dtype=torch.bool).tril()
+    mask[:, 0] = False
+    sk[:, 0], sv[:, 0] = float("nan"), float("nan")
+    pl = torch.randn(b, s, hq, generator=g)
+    pl[:, :, 0], po[:, :, 0] = float("-inf"), float("nan")
+    out = torch.empty(b, s, hq, d, dtype=torch.float16, device="cuda")
+    args = cabi.tree_suffix_args_from_tensors(*[x.cuda() for x in (q, sk, sv, mask, po, pl)], out, 0.2)
+    cabi.tree_suffix_merge(args, torch.cuda.current_stream().cuda_stream)
+    kf, vf = (x.double().nan_to_num(0.0).repeat_interleave(hq // hkv, 2) for x in (sk, sv))
+    w = torch.exp((q.double()[:, :, :, None] * kf.permute(0, 2, 1, 3)[:, None]).sum(-1) * 0.2) * mask[None, :, None]
+    wp = torch.exp(pl.double())
+    num = (w[..., None] * vf.permute(0, 2, 1, 3)[:, None]).sum(3) + wp[..., None] * po.double().nan_to_num(0.0)
+    den = (w.sum(3) + wp)[..., None]
+    exp = torch.where(den > 0, num / den, torch.zeros_like(num))
+    # half an ulp of fp16 (2^-12 relative), doubled, plus 1e-3 for the fp32 arithmetic
+    assert torch.all((out.double().cpu() - exp).abs() <= 2.0 ** -11 * exp.abs() + 1e-3)
+
+
 def _hybrid_inputs(batch, hq, hkv, d, cached, draft, seed, kv=torch.bfloat16):
     kc, vc, ks, vs, table, pk, pv = _paged_prefix(batch, hkv, d, cached, kv, seed=seed)
     g = torch.Generator().manual_seed(seed + 1)
