@@ -436,7 +436,7 @@ __device__ __forceinline__ void publish_scale(float *out, int h, float amax, boo
 // lane owns eight contiguous dims, D/8 lanes a row, scale_rows rows of K and
 // V in flight per lane), and every lane group keeps one head, so the maxima stay
 // in registers until the workgroup's LDS fold.  blockIdx.y: block of hb heads.
-// 16K tokens of 4 KV heads at head_dim 128 (38 MB): 13.5 us, 2.8 TB/s, where one
+// 16K tokens of 4 KV heads at head_dim 128 (38 MB): 12.3 us, 3.1 TB/s, where one
 // workgroup per (head, K or V) took 3158 us.  256 workgroups of 16 waves, the
 // whole chunk in flight at once; 1024 of 4 waves 22.3 us per call and 512 of 8
 // 17.0 us (more atomics on one line), against 15.1 us; without the atomics 13.2.
@@ -461,29 +461,35 @@ __global__ __launch_bounds__(kScaleThreads) void kv_amax8(Params p, float *k_out
   const int head = blockIdx.y * hb + (group - off * hb);
   const bool used = g < rpw && off < tpp && head < p.hkv;
   const int64_t t_end = min((int64_t)p.tokens, ((int64_t)blockIdx.x + 1) * chunk);
-  const T *kbase = reinterpret_cast<const T *>(p.k) + (int64_t)head * p.k_sh + e0;
-  const T *vbase = reinterpret_cast<const T *>(p.v) + (int64_t)head * p.v_sh + e0;
+  const int64_t held = min(head, p.hkv - 1);
+  const T *kbase = reinterpret_cast<const T *>(p.k) + held * p.k_sh + e0;
+  const T *vbase = reinterpret_cast<const T *>(p.v) + held * p.v_sh + e0;
   // the neox partner's words, from the lane half/8 away in the same row
   const int src = (p.neox && rot_lane) ? g * lpr + (e0 < half ? l + (half >> 3) : l - (half >> 3)) : lane;
   float mk = 0.0f, mv = 0.0f;
   for (int64_t t0 = (int64_t)blockIdx.x * chunk; t0 < t_end; t0 += kRows * tpp) {  // uniform: every lane shuffles
     i32x4 kw[kRows], vw[kRows];
-    int64_t pos[kRows];
-    bool live[kRows];
+    int64_t pos[kRows], slot[kRows];
+    // Every load of the pass without a branch (past the chunk: its last token again),
+    // positions and slots first: a slot compared where it is loaded, in a branch,
+    // waits there for all loads so far (16K tokens of 4 heads: 13.5 -> 12.3 us).
 #pragma unroll
     for (int u = 0; u < kRows; ++u) {
-      const int64_t t = t0 + (int64_t)u * tpp + off;
-      live[u] = used && t < t_end;
-      kw[u] = vw[u] = i32x4{0, 0, 0, 0};
-      pos[u] = 0;
-      if (live[u]) {
-        kw[u] = *reinterpret_cast<const i32x4 *>(kbase + t * p.k_st);
-        vw[u] = *reinterpret_cast<const i32x4 *>(vbase + t * p.v_st);
-        pos[u] = p.pos[t];
-        const int64_t slot = p.slots[t];
-        live[u] = slot >= 0 && (slot >> 4) < p.num_pages;  // else not stored
-      }
+      const int64_t t = min(t0 + (int64_t)u * tpp + off, t_end - 1);
+      pos[u] = p.pos[t];
+      slot[u] = p.slots[t];
     }
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int64_t t = min(t0 + (int64_t)u * tpp + off, t_end - 1);
+      kw[u] = *reinterpret_cast<const i32x4 *>(kbase + t * p.k_st);
+      vw[u] = *reinterpret_cast<const i32x4 *>(vbase + t * p.v_st);
+    }
+    bool live[kRows];
+#pragma unroll
+    for (int u = 0; u < kRows; ++u)
+      live[u] = used && t0 + (int64_t)u * tpp + off < t_end && slot[u] >= 0 &&
+                (slot[u] >> 4) < p.num_pages;  // else not stored
     CosSin<CS> cs[kRows];
 #pragma unroll
     for (int u = 0; u < kRows; ++u)
