@@ -287,36 +287,37 @@ __global__ __launch_bounds__(256) void kv_rope_write8(Params p, uint32_t rows_q,
   T *row[ROWS];
   int head[ROWS];
   bool live[ROWS], is_k[ROWS];
-  // Positions first: the cos/sin loads wait for them alone, with the rows in flight
-  // (16K tokens, 32 heads of 128: 63.3 -> 62.1 us; small calls do not change).
-  int64_t tok[ROWS];
 #pragma unroll
   for (int u = 0; u < ROWS; ++u) {
     const uint32_t r = first + (uint32_t)((u * 4 + wave) * rpw + g);
     live[u] = g < rpw && r < rows_all;
     is_k[u] = r >= rows_q;
-    const uint32_t n = is_k[u] ? r - rows_q : r, heads = (uint32_t)(is_k[u] ? p.hkv : p.hq);
-    const uint32_t t = n / heads;
-    tok[u] = t;
-    head[u] = (int)(n - t * heads);
-    pos[u] = 0;
-    if (live[u] && rot_lane) pos[u] = p.pos[t];
-  }
-#pragma unroll
-  for (int u = 0; u < ROWS; ++u) {
-    row[u] = is_k[u] ? reinterpret_cast<T *>(p.k) + tok[u] * p.k_st + (int64_t)head[u] * p.k_sh
-                     : reinterpret_cast<T *>(p.q) + tok[u] * p.q_st + (int64_t)head[u] * p.q_sh;
-    if (!live[u]) continue;
-    xw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(row[u] + e0));
-    if (is_k[u]) {
-      vw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(
-          reinterpret_cast<const T *>(p.v) + tok[u] * p.v_st + (int64_t)head[u] * p.v_sh + e0));
-      slot[u] = p.slots[tok[u]];
-      if constexpr (CT == 0) {
-        ksc[u] = p.k_scale_ph ? p.k_scale_ph[head[u]] : p.k_scale;
-        vsc[u] = p.v_scale_ph ? p.v_scale_ph[head[u]] : p.v_scale;
+    int64_t t = 0;
+    int h = 0;
+    if (live[u]) {
+      if (!is_k[u]) {
+        const uint32_t q = r / (uint32_t)p.hq;
+        t = q;
+        h = (int)(r - q * (uint32_t)p.hq);
+        row[u] = reinterpret_cast<T *>(p.q) + t * p.q_st + (int64_t)h * p.q_sh;
+      } else {
+        const uint32_t rk = r - rows_q;
+        const uint32_t q = rk / (uint32_t)p.hkv;
+        t = q;
+        h = (int)(rk - q * (uint32_t)p.hkv);
+        row[u] = reinterpret_cast<T *>(p.k) + t * p.k_st + (int64_t)h * p.k_sh;
+        vw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(reinterpret_cast<const T *>(p.v) + t * p.v_st +
+                                                 (int64_t)h * p.v_sh + e0));
+        slot[u] = p.slots[t];
+        if constexpr (CT == 0) {
+          ksc[u] = p.k_scale_ph ? p.k_scale_ph[h] : p.k_scale;
+          vsc[u] = p.v_scale_ph ? p.v_scale_ph[h] : p.v_scale;
+        }
       }
+      xw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(row[u] + e0));
+      pos[u] = p.pos[t];
     }
+    head[u] = h;
   }
   // ---- cos / sin of the lanes' dims ----
   CosSin<CS> cs[ROWS];
