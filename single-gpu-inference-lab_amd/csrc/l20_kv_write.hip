@@ -3,8 +3,8 @@
 //
 //  kv_rope_write8<T, CT, CS, ROWS>   the fast path: every Q and K head row of the
 //    call is one row of the work; a lane owns eight contiguous dims (16-byte
-//    loads and stores), D/8 lanes a row, and each lane takes ROWS rows (one in
-//    small calls, else two) with all their loads issued before any arithmetic;
+//    loads and stores), D/8 lanes a row, and each lane takes ROWS rows (one or
+//    two by the call's size) with all their loads issued before any arithmetic;
 //    row numbers are 32-bit (the 64-bit divisions cost a small call ~0.1 us).  A neox pair partner lies
 //    half/8 lanes away in the same row and is exchanged with a lane shuffle;
 //    cos and sin arrive as 8 (neox) or 4 (interleaved) consecutive values.
@@ -721,15 +721,21 @@ void launch_fast_rows(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uin
     hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
 }
 
-// One row per lane while the workgroups of one fit the chip at once (8 per CU: a
-// small call is one chain of dependent loads, and a second row only lengthens
-// it), else two.  32 heads of 128, fp8 cache, us per call with one and two, in a
-// graph: 16 tokens 3.44, 4.30; 128 tokens 4.01, 4.89; 1024 (2048 workgroups of
-// one) 6.21, 6.61; 1500 8.81, 8.30; 16384 64.8, 64.2.
+// Rows per lane.  A call is a chain of dependent loads, so what decides is whether
+// its workgroups are on the chip at once: 8 a CU of one row per lane (2048), 6 of
+// two (1536, the rows of 3072 of one).  Up to 2048 workgroups one row, up to 3072
+// two, beyond them one again (the shorter last round), until the stream is long
+// enough for the loads in flight to count: 16384 with fp8 caches, whose quantiser
+// needs the waves, 4096 with 16-bit ones.  us per call with one and two rows, in a
+// graph, by workgroups of one row, 28 + 4 heads of 128 with an fp8 and a bf16 cache:
+// 1024 4.2, 5.0 and 3.8, 4.2; 1900 5.2, 6.0 and 5.5, 5.6; 2100 7.0, 6.5 and 6.5, 6.2;
+// 2800 7.9, 7.3 and 7.5, 7.3; 3300 8.5, 10.1 and 8.4, 9.5; 4000 10.1, 11.0 and 10.1,
+// 10.4; 7000 16.7, 17.7 and 16.7, 16.4; 16000 33.6, 34.7 and 34.1, 34.0; 32000 63.4,
+// 63.1 and 63.0, 63.6.  8 + 1 heads, bf16 cache: 9216 22.0, 21.1.
 template <typename T, int CT>
 void launch_fast(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uint32_t rows_all, hipStream_t s) {
   const int64_t one = ((int64_t)rows_all + 4 * (64 / (p.d / 8)) - 1) / (4 * (64 / (p.d / 8)));
-  if (one <= 2048) launch_fast_rows<T, CT, 1>(p, cs_dtype, rows_q, rows_all, s);
+  if (one <= 2048 || (one > 3072 && one <= (CT == 0 ? 16384 : 4096))) launch_fast_rows<T, CT, 1>(p, cs_dtype, rows_q, rows_all, s);
   else launch_fast_rows<T, CT, 2>(p, cs_dtype, rows_q, rows_all, s);
 }
 

@@ -244,29 +244,35 @@ def test_fp8_scales_match_oracle(per_head):
     np.testing.assert_array_equal(_np(k), _np(c["k"]))  # the scale pass leaves K untouched
 
 
-@pytest.mark.parametrize("tokens", [1, 1023, 1025, 2731])
-def test_one_and_two_rows_per_lane(tokens):
-    """Both sides of the rows-per-lane rule (2048 workgroups: 1024 tokens of 32 head rows
-    of 128), the last workgroup full and not: bit exact against the producer's oracle."""
+@pytest.mark.parametrize("fp8", [True, False], ids=["fp8", "bf16"])
+@pytest.mark.parametrize("tokens", [1, 1023, 1025, 1536, 1537, 2048, 2049, 2731, 8192, 8193])
+def test_one_and_two_rows_per_lane(tokens, fp8):
+    """Both sides of each line of the rows-per-lane rule (2048, 3072 and, by the cache type,
+    4096 or 16384 workgroups: 1024, 1536, 2048 and 8192 tokens of 32 head rows of 128), the
+    last workgroup full and not: bit exact against the producer's oracle."""
     from oracle import kv_write_ref as kw
     import l20_rope_kv
 
     c = _case(max(tokens, 2), 28, 4, 128, 128, torch.bfloat16, torch.bfloat16, seed=tokens)
     c = {k: (v[:tokens] if isinstance(v, torch.Tensor) and k != "cs" else v) for k, v in c.items()}
     q, k = c["q"].cuda(), c["k"].cuda()
-    kc = torch.zeros(c["pages"], 16, 4, 128, dtype=torch.float8_e4m3fn).cuda()
+    kc = torch.zeros(c["pages"], 16, 4, 128, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16).cuda()
     vc = kc.clone()
+    scales = (0.02, 0.03) if fp8 else (1.0, 1.0)
     l20_rope_kv.l20_rope_and_cache(q, k, c["v"].cuda(), c["pos"].cuda(), c["cs"].cuda(), True, kc, vc,
-                                   c["slots"].cuda(), k_scale=0.02, v_scale=0.03)
+                                   c["slots"].cuda(), k_scale=scales[0], v_scale=scales[1])
     cs = _np(c["cs"])[c["pos"].numpy()]
     k_rot = kw.round_bf16(kw.rope(_np(c["k"]), cs, 128, True))
     np.testing.assert_array_equal(_np(q), kw.round_bf16(kw.rope(_np(c["q"]), cs, 128, True)))
     np.testing.assert_array_equal(_np(k), k_rot)
     stored = c["slots"].numpy()
     live = stored >= 0
-    for cache, rows, scale in ((kc, k_rot, 0.02), (vc, _np(c["v"]), 0.03)):
-        got = cache.view(torch.uint8).cpu().numpy().reshape(-1, 4, 128)
-        np.testing.assert_array_equal(got[stored[live]], kw.quantize_rows(rows[live], np.float32(scale)))
+    for cache, rows, scale in ((kc, k_rot, scales[0]), (vc, _np(c["v"]), scales[1])):
+        if fp8:
+            got = cache.view(torch.uint8).cpu().numpy().reshape(-1, 4, 128)
+            np.testing.assert_array_equal(got[stored[live]], kw.quantize_rows(rows[live], np.float32(scale)))
+        else:
+            np.testing.assert_array_equal(_np(cache).reshape(-1, 4, 128)[stored[live]], rows[live])
 
 
 @pytest.mark.parametrize("per_head", [True, False])
