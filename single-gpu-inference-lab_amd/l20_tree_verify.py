@@ -366,6 +366,8 @@ def hybrid_tree_attention_paged_prefix(
             raise ValueError("contiguous_pages=True requires page_base=[B]")
         if page_base.ndim != 1 or page_base.shape[0] != batch:
             raise ValueError("page_base must have shape [B]")
+        if page_base.device != query.device:
+            raise RuntimeError("page_base must be on the query's device")
     scale = head_dim ** -0.5 if softmax_scale is None else float(softmax_scale)
     ws = _as_workspace(workspace, query)
     dev = query.device

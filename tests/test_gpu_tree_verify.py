@@ -363,6 +363,18 @@ def _hybrid_inputs(batch, hq, hkv, d, cached, draft, seed, kv=torch.bfloat16):
     return dict(query=query, kc=kc, vc=vc, ks=ks, vs=vs, table=table, sk=sk, sv=sv, mask=mask, pk=pk, pv=pv)
 
 
+def test_hybrid_page_base_on_another_device_is_refused():
+    """A host page_base is an error, not a hidden copy (one and several packed chunks)."""
+    import l20_tree_verify as tv
+
+    for draft, hq, hkv in ((4, 8, 2), (8, 28, 4)):
+        x = _hybrid_inputs(2, hq, hkv, 128, 100, draft, seed=5)
+        with pytest.raises(RuntimeError, match="page_base"):
+            tv.hybrid_tree_attention_paged_prefix(x["query"], x["kc"], x["vc"], x["sk"], x["sv"], x["table"], x["mask"],
+                                                  100, contiguous_pages=True,
+                                                  page_base=torch.zeros(2, dtype=torch.int32))
+
+
 @pytest.mark.parametrize("draft,hq,hkv", [(8, 28, 4), (5, 8, 2)])  # two packed chunks; one padded chunk
 def test_hybrid_warmed_workspace_allocates_nothing_and_replays_in_a_graph(draft, hq, hkv):
     import l20_tree_verify as tv
