@@ -424,8 +424,8 @@ __global__ void kv_scales_init(float *k_scales, float *v_scales, int hkv) {
 
 // One workgroup's maxima -> the scales.  A positive float orders as its bits.
 // single: the only workgroup of the call, which stores (no kv_scales_init ran).
-// All of a workgroup's K (V) atomics leave in one instruction over consecutive
-// words: device-scope atomics on one line are served one request at a time.
+// Consecutive lanes hold consecutive heads, so up to 64 heads leave in one instruction
+// over consecutive words: device-scope atomics on one line are served one request at a time.
 __device__ __forceinline__ void publish_scale(float *out, int h, float amax, bool single) {
   const float s = scale_of(amax);
   if (single) out[h] = s;
@@ -438,9 +438,10 @@ __device__ __forceinline__ void publish_scale(float *out, int h, float amax, boo
 // V in flight per lane), and every lane group keeps one head, so the maxima stay
 // in registers until the workgroup's LDS fold.  blockIdx.y: block of hb heads.
 // 16K tokens of 4 KV heads at head_dim 128 (38 MB): 12.3 us, 3.1 TB/s, where one
-// workgroup per (head, K or V) took 3158 us.  256 workgroups of 16 waves, the
-// whole chunk in flight at once; 1024 of 4 waves 22.3 us per call and 512 of 8
-// 17.0 us (more atomics on one line), against 15.1 us; without the atomics 13.2.
+// workgroup per (head, K or V) took 3158 us; 13.0 us per call with the initialising
+// launch.  256 workgroups of 16 waves, the whole chunk in flight at once.  Per call
+// with an earlier order of its loads: 15.1 us, 13.2 without the atomics, 512
+// workgroups of 8 waves 17.0, 1024 of 4 22.3 (more atomics on one line).
 template <typename T, int CS>
 __global__ __launch_bounds__(kScaleThreads) void kv_amax8(Params p, float *k_out, float *v_out, int hb, int chunk,
                                                          int per_head, int single) {
@@ -822,8 +823,9 @@ int32_t l20_pd_kv_fp8_scales(const l20_pd_kv_write_args *a, float *k_scales, flo
   // At least 32 dims (the fold's LDS rows): smaller heads take the general path.
   const bool fast = a->num_tokens > 0 && p.d >= 32 && fast_path_ok(b);
   // Fast path: one pass of the grid where it can be (16K tokens, 4 KV heads:
-  // 256 workgroups of 64 tokens), never more workgroups than CUs, since their
-  // atomics on the scales' line are served one at a time (~11 ns each).
+  // 256 workgroups of 64 tokens), at most 256 workgroups (an MI355X's CUs) for each
+  // block of hb heads, since the atomics on one line of scales are served one at a
+  // time (~11 ns each).
   const int groups = (l20kv::kScaleThreads / 64) * (fast ? 64 / (p.d / 8) : 1);
   const int hb = std::min(p.hkv, groups);
   const int step = l20kv::scale_rows(p.cs_dtype) * (groups / hb);  // tokens per workgroup and loop pass

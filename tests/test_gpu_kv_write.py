@@ -278,9 +278,10 @@ def test_one_and_two_rows_per_lane(tokens, fp8):
 @pytest.mark.parametrize("per_head", [True, False])
 @pytest.mark.parametrize("tokens,hkv,d,rot,neox,cs,offset", [
     (1, 4, 128, 128, True, torch.bfloat16, 0),      # one workgroup
-    (33, 1, 128, 128, True, torch.float32, 0),      # one row past the first pass
+    (33, 1, 128, 128, True, torch.float32, 0),      # a fraction of one pass
+    (129, 1, 128, 128, True, torch.float32, 0),     # one row past a pass: a second workgroup
     (127, 3, 64, 32, False, torch.float16, 0),      # lane groups left over, interleaved, partial rotary
-    (5000, 8, 128, 64, True, torch.bfloat16, 0),    # several passes per workgroup
+    (5000, 8, 128, 64, True, torch.bfloat16, 0),    # many workgroups of one pass
     (777, 5, 96, 96, True, torch.bfloat16, 0),      # 12 lanes a row
     (65, 80, 256, 256, True, torch.bfloat16, 0),    # more heads than lane groups of a workgroup
     (300, 4, 16, 16, True, torch.bfloat16, 0),      # head_dim below the fast path's
@@ -312,6 +313,34 @@ def test_fp8_scales_over_shapes(tokens, hkv, d, rot, neox, cs, offset, per_head)
     want = [kw.fp8_scales(k_rot, per_head), kw.fp8_scales(_np(c["v"])[stored], per_head)]
     for got, w in zip((ks, vs), want):
         np.testing.assert_array_equal(got.cpu().numpy(), np.broadcast_to(w, hkv))
+
+
+@pytest.mark.parametrize("tokens,hkv,d,rot,cs,peak", [
+    (1100, 32, 256, 256, torch.bfloat16, 1095),   # passes of 4 tokens, two a workgroup
+    (2051, 32, 256, 256, torch.bfloat16, 2050),   # three, the last workgroup's third of 3 tokens
+    (9001, 8, 128, 128, torch.bfloat16, 9000),    # passes of 32, the last one of 9 tokens
+    (5001, 8, 128, 64, torch.float32, 4991),      # an fp32 table: passes of 16
+])
+def test_fp8_scales_over_several_passes(tokens, hkv, d, rot, cs, peak):
+    """More tokens than 256 workgroups take in one pass each: maxima carried from pass to
+    pass, the largest K and V in a row of a later pass, and (per head) in every other row."""
+    from oracle import kv_write_ref as kw
+    import l20_rope_kv
+
+    c = _case(tokens, 2 * hkv, hkv, d, rot, torch.bfloat16, cs, seed=tokens)
+    slots = c["slots"].clone()
+    slots[peak] = 3
+    for head in range(0, hkv, 2):
+        c["k"][peak, head, head % d] = 40.0 + head
+        c["v"][peak, head, (3 * head) % d] = -50.0 - head
+    kc = torch.zeros(c["pages"], 16, hkv, d, dtype=torch.float8_e4m3fn).cuda()
+    stored = (slots >= 0).numpy()
+    k_rot = kw.round_bf16(kw.rope(_np(c["k"]), _np(c["cs"])[c["pos"].numpy()], rot, True))[stored]
+    for per_head in (True, False):
+        ks, vs = l20_rope_kv.l20_kv_fp8_scales(c["k"].cuda(), c["v"].cuda(), c["pos"].cuda(), c["cs"].cuda(), True, kc,
+                                               kc.clone(), slots.cuda(), per_head=per_head)
+        for got, rows in ((ks, k_rot), (vs, _np(c["v"])[stored])):
+            np.testing.assert_array_equal(got.cpu().numpy(), np.broadcast_to(kw.fp8_scales(rows, per_head), hkv))
 
 
 def test_produced_fp8_cache_feeds_the_decode_op():
