@@ -337,11 +337,8 @@ def run_decode(args, mode):
     # merge): that kernel is then the call, and the roofline times it as such.
     # Batches whose 512-token splits fill the CUs once run the partial stage
     # as that kernel's split mode (then the merge): the roofline times it.
-    path = cabi.launch_path(calls[0][0], lib)
-    single = path == 1
-    # The other workloads' partial stage: pd_units, except with 16-bit caches (8192
-    # units at most here, past that kernel's limit for them).
-    kernel = "pd_fp8_fused" if path else "pd_units" if elem == 1 else "pd_fp8_partial"
+    single = cabi.launch_path(calls[0][0], lib) == 1
+    kernel = cabi.partial_kernel(calls[0][0], lib)
     kernel_fn = cabi.split_out if single else cabi.partial
 
     settle_calls, settle_ms = settle(lambda i: cabi.split_out(calls[i % n_sets][0], h, lib), args.settle_ms)

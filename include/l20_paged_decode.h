@@ -222,6 +222,15 @@ int32_t l20_pd_set_spin_limit(uint32_t polls);
  * than) half of them. */
 int32_t l20_pd_single_launch(const l20_pd_fp8_args *args);
 
+/* The kernel of that call's partial stage on the current device: 1 and 2 as
+ * l20_pd_single_launch, 3 the kernel that spreads (sequence, split, KV head)
+ * units evenly over the CUs (pd_units), 0 the persistent work-queue kernel;
+ * -(error code) when the arguments fail l20_pd_fp8_e4m3_check.  Host only, no
+ * reference counterpart.  Of the calls that l20_pd_single_launch gives 0 for,
+ * pd_units takes those of at most 256 sequences, except 16-bit caches beyond 16
+ * units per CU and head_dim 64 beyond 32 (batch x num_kv_heads x splits). */
+int32_t l20_pd_partial_kernel(const l20_pd_fp8_args *args);
+
 /* Sets every work-queue counter of the current device to `value` (after a
  * device synchronize), as a launch that gave up mid-way or shared a slot with
  * another leaves it.  A test hook with no reference counterpart: with a value

@@ -3515,6 +3515,11 @@ int32_t l20_pd_set_spin_limit(uint32_t polls) {
 }
 
 int32_t l20_pd_single_launch(const l20_pd_fp8_args *a) {
+  const int32_t kernel = l20_pd_partial_kernel(a);
+  return kernel == 3 ? 0 : kernel;
+}
+
+int32_t l20_pd_partial_kernel(const l20_pd_fp8_args *a) {
   g_last_error[0] = '\0';
   const int32_t rc = check_args(a);
   if (rc != L20_PD_OK) return -rc;
@@ -3523,7 +3528,9 @@ int32_t l20_pd_single_launch(const l20_pd_fp8_args *a) {
   const int n_s = l20_pd_num_splits(a->max_seq_len, a->split_size);
   const int nqt = (a->num_q_heads / a->num_kv_heads * a->q_len + 15) / 16;
   const l20pd::PartialParams pp = partial_params(*a, n_s);
-  return fused_fits(*a, pp, nqt, kv16) ? 1 : fused_split_fits(*a, pp, nqt, kv16) ? 2 : 0;
+  if (fused_fits(*a, pp, nqt, kv16)) return 1;
+  if (fused_split_fits(*a, pp, nqt, kv16)) return 2;
+  return units_fit(*a, pp, nqt, kv16) ? 3 : 0;
 }
 
 int32_t l20_pd_set_queue_counters(uint64_t value) {

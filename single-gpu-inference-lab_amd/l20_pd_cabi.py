@@ -33,6 +33,7 @@ EXPORTED = (
     "l20_pd_set_spin_limit",
     "l20_pd_set_queue_counters",
     "l20_pd_single_launch",
+    "l20_pd_partial_kernel",
     "l20_pd_split_out",
     "l20_pd_fp8_e4m3_partial",
     "l20_pd_fp8_e4m3_merge",
@@ -144,8 +145,9 @@ def load(path: Optional[Path] = None) -> ctypes.CDLL:
     lib.l20_pd_set_spin_limit.restype = _i32
     lib.l20_pd_set_queue_counters.argtypes = [ctypes.c_uint64]
     lib.l20_pd_set_queue_counters.restype = _i32
-    lib.l20_pd_single_launch.argtypes = [ctypes.POINTER(L20PdFp8Args)]
-    lib.l20_pd_single_launch.restype = _i32
+    for name in ("l20_pd_single_launch", "l20_pd_partial_kernel"):
+        getattr(lib, name).argtypes = [args_p]
+        getattr(lib, name).restype = _i32
     lib.l20_pd_default_split_size.argtypes = [_i32, _i32, _i32, _i32]
     lib.l20_pd_default_split_size.restype = _i32
     lib.l20_pd_fp8_e4m3_dequant_f32.argtypes = [_vp, _vp, _i64, _f32, _vp]
@@ -324,6 +326,20 @@ def launch_path(args: L20PdFp8Args, lib: Optional[ctypes.CDLL] = None) -> int:
     if rc < 0:
         raise RuntimeError(last_error(lib))
     return int(rc)
+
+
+# l20_pd_partial_kernel's codes (1 and 2 are one kernel: whole sequences, splits).
+PARTIAL_KERNELS = {0: "pd_fp8_partial", 1: "pd_fp8_fused", 2: "pd_fp8_fused", 3: "pd_units"}
+
+
+def partial_kernel(args: L20PdFp8Args, lib: Optional[ctypes.CDLL] = None) -> str:
+    """``l20_pd_partial_kernel`` by name: the kernel of the call's partial stage (or,
+    for a single launch, of the whole call)."""
+    lib = lib or load()
+    rc = lib.l20_pd_partial_kernel(ctypes.byref(args))
+    if rc < 0:
+        raise RuntimeError(last_error(lib))
+    return PARTIAL_KERNELS[rc]
 
 
 def set_queue_counters(value: int, lib: Optional[ctypes.CDLL] = None) -> None:

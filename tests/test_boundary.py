@@ -249,6 +249,42 @@ def _with_split(a, split):
     return a
 
 
+def test_partial_kernel_rule(monkeypatch):
+    """l20_pd_partial_kernel names the partial stage's kernel; of l20_pd_single_launch's 0
+    it tells pd_units (at most 256 sequences; with 16-bit caches at most 16 units per CU,
+    at head_dim 64 at most 32; 256 CUs here, no GPU) from the persistent kernel."""
+    for name in ("L20_PD_FUSED", "L20_PD_FUSED_SPLIT", "L20_PD_UNITS"):
+        monkeypatch.delenv(name, raising=False)
+    a = valid_args()  # 28 query / 4 KV heads, 8 x 1024 tokens
+    assert cabi.partial_kernel(a) == "pd_fp8_fused" and cabi.launch_path(a) == 1
+    a.max_seq_len, a.bt_stride_row, a.bt_max_pages = 2048, 128, 128
+    _with_split(a, 512)
+    a.batch = 16
+    assert cabi.partial_kernel(a) == "pd_fp8_fused" and cabi.launch_path(a) == 2
+    for batch, kernel in ((17, "pd_units"), (256, "pd_units"), (257, "pd_fp8_partial")):
+        a.batch = batch
+        assert cabi.partial_kernel(a) == kernel and cabi.launch_path(a) == 0
+    a.batch = 256  # 4096 units, 8192 at 256-token splits
+    a.kv_dtype = cabi.L20_PD_KV_BF16
+    assert cabi.partial_kernel(a) == "pd_units"
+    _with_split(a, 256)
+    assert cabi.partial_kernel(a) == "pd_fp8_partial"
+    a.kv_dtype = cabi.L20_PD_KV_FP8_E4M3
+    assert cabi.partial_kernel(a) == "pd_units"
+    a.head_dim = 64
+    assert cabi.partial_kernel(a) == "pd_units"
+    _with_split(a, 128)  # 16384
+    assert cabi.partial_kernel(a) == "pd_fp8_partial"
+    monkeypatch.setenv("L20_PD_UNITS", "1")
+    assert cabi.partial_kernel(a) == "pd_units"
+    monkeypatch.setenv("L20_PD_UNITS", "0")
+    a.batch = 17
+    assert cabi.partial_kernel(a) == "pd_fp8_partial"
+    a.split_size = 100
+    with pytest.raises(RuntimeError, match="split_size"):
+        cabi.partial_kernel(a)
+
+
 def test_split_mode_rule(monkeypatch):
     """l20_pd_single_launch returns 2 when the partial stage runs as the
     single-launch kernel's split mode (one workgroup per (split, sequence, KV

@@ -14,7 +14,7 @@ import pytest
 import torch
 
 import pd_helpers as H
-from test_gpu_fused_split import _run
+from test_gpu_fused_split import _run as _run_call
 from test_gpu_random_sweep import draw, run_case
 
 pytestmark = pytest.mark.gpu
@@ -27,6 +27,28 @@ def _units(monkeypatch):
     monkeypatch.setenv("L20_PD_FUSED", "0")
     monkeypatch.setenv("L20_PD_FUSED_SPLIT", "2")  # neither the split mode nor the persistent kernel
     monkeypatch.setenv("L20_PD_UNITS", "1")
+
+
+@pytest.fixture
+def kernels(monkeypatch):
+    """The partial kernel of every call made through the C ABI, as the library names it."""
+    import l20_pd_cabi as cabi
+
+    ran, split_out = [], cabi.split_out
+
+    def named(args, *rest):
+        ran.append(cabi.partial_kernel(args))
+        return split_out(args, *rest)
+
+    monkeypatch.setattr(cabi, "split_out", named)
+    return ran
+
+
+def _run(inp, split, pdt, kernels, kernel="pd_units"):
+    """One call through the C ABI, on ``kernel``."""
+    out, lse, path = _run_call(inp, split, pdt)
+    assert path == 0 and kernels[-1] == kernel
+    return out, lse
 
 
 CASES = [
@@ -47,25 +69,24 @@ CASES = [
 
 
 @pytest.mark.parametrize("case", CASES, ids=[c[0] for c in CASES])
-def test_units_match_oracle(case, monkeypatch):
+def test_units_match_oracle(case, monkeypatch, kernels):
     name, batch, hq, hkv, d, lens, q_len, per_head, fp8, page, split, pdt, groups = case
     if groups:
         monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", str(groups))
     inp = H.make_synthetic(batch, hq, hkv, d, lens, q_len=q_len, per_head=per_head, fp8=fp8, page=page,
                            seed=zlib.crc32(name.encode()) % 1000, garbage_tail=True)
-    out, lse, path = _run(inp, split, PDT[pdt])
-    assert path == 0
+    out, lse = _run(inp, split, PDT[pdt], kernels)
     H.compare(out, lse, *H.run_oracle(inp))
 
 
 @pytest.mark.parametrize("batch", [65, 256])
-def test_units_many_sequences(batch, monkeypatch):
+def test_units_many_sequences(batch, monkeypatch, kernels):
     """Lanes hold two and four sequences' lengths."""
     monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", "11")
     rng = np.random.default_rng(batch)
     lens = [int(x) for x in rng.choice([0, 1, 63, 64, 65, 200, 400], size=batch)]
     inp = H.make_synthetic(batch, 4, 2, 64, lens, seed=batch, garbage_tail=True)
-    out, lse, _ = _run(inp, 64, torch.float32)
+    out, lse = _run(inp, 64, torch.float32, kernels)
     H.compare(out, lse, *H.run_oracle(inp))
 
 
@@ -78,9 +99,9 @@ def test_units_random_shape(case, groups, monkeypatch):
     run_case(c)
 
 
-def test_units_graph_replays_match_eager():
+def test_units_graph_replays_match_eager(kernels):
     inp = H.make_synthetic(6, 28, 4, 128, [900, 31, 1500, 0, 512, 77], seed=5)
-    ref, ref_lse, _ = _run(inp, 256, torch.float32)
+    ref, _ = _run(inp, 256, torch.float32, kernels)
     q = inp["query"]
     po, pm, ps = H.workspace(inp, 256, torch.float32)
     out = torch.empty_like(q)
@@ -108,16 +129,15 @@ def test_units_graph_replays_match_eager():
         assert torch.equal(out, ref)
 
 
-def test_library_takes_the_units_kernel(monkeypatch):
+def test_library_takes_the_units_kernel(monkeypatch, kernels):
     """By the library's own rule (no override), bitwise the forced call's result; a batch
     past the lengths a wave holds runs the persistent kernel, to the oracle all the same."""
     inp = H.make_synthetic(24, 16, 2, 128, [40 + 57 * i for i in range(24)], seed=3)
-    forced, forced_lse, _ = _run(inp, 256, torch.float32)
+    forced, forced_lse = _run(inp, 256, torch.float32, kernels)
     for name in ("L20_PD_FUSED", "L20_PD_FUSED_SPLIT", "L20_PD_UNITS"):
         monkeypatch.delenv(name, raising=False)
-    out, lse, path = _run(inp, 256, torch.float32)
-    assert path == 0
+    out, lse = _run(inp, 256, torch.float32, kernels)
     assert torch.equal(out, forced) and torch.equal(lse, forced_lse)
     big = H.make_synthetic(257, 4, 2, 64, [1 + 7 * (i % 90) for i in range(257)], seed=4)
-    out, lse, _ = _run(big, 64, torch.float32)
+    out, lse = _run(big, 64, torch.float32, kernels, kernel="pd_fp8_partial")
     H.compare(out, lse, *H.run_oracle(big))
