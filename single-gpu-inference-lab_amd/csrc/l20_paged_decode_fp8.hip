@@ -3050,8 +3050,7 @@ hipError_t launch_units(const l20pd::PartialParams &pp, int head_dim, int nqt, i
 // the host can see): 128 lognormal sequences, 4 KV heads 81.8 against 83.2 us per
 // call (8192 units at most), 64 of them 45.8 against 44.4 (4096).  At head_dim 64,
 // beyond 32: 200 x uniform to 3000, 8 KV heads 88.4 against 91.0 (9600), 100 of
-// them 53.6 against 46.5 (4800).  L20_PD_FUSED_SPLIT=0 keeps every partial stage on
-// the persistent kernel, L20_PD_UNITS=0/1 overrides the size rule (tests and
+// them 53.6 against 46.5 (4800).  L20_PD_UNITS=0/1 overrides the size rule (tests and
 // measurement).
 bool units_fit(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, int nqt, bool kv16) {
   if (nqt > 2 || a.batch > l20pd::kUnitMaxBatch) return false;
@@ -3060,8 +3059,6 @@ bool units_fit(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, int nqt
   if (units >= ((int64_t)1 << 27) || units * a.num_kv_heads >= ((int64_t)1 << 32) ||
       ((int64_t)pp.l_cap + a.split_size) * a.split_size >= ((int64_t)1 << 32))
     return false;
-  if (const char *env = getenv("L20_PD_FUSED_SPLIT"))
-    if (env[0] == '0') return false;
   if (const char *env = getenv("L20_PD_UNITS")) return env[0] == '1';
   const int64_t per_cu = kv16 ? 16 : a.head_dim == 64 ? 32 : INT64_MAX / 65536;
   return units <= per_cu * device_cus();

@@ -28,6 +28,25 @@ def _split_path_by_default(monkeypatch):
     the single launch ask for it (L20_PD_FUSED=1) or for the library's choice
     (the variable removed).  Likewise the single-launch kernel's split mode
     (512-token splits whose triples fill the CUs once) is off unless a test
-    asks for it (L20_PD_FUSED_SPLIT=1) or for the library's choice."""
+    asks for it (L20_PD_FUSED_SPLIT=1) or for the library's choice.  Which of the
+    two partial kernels then runs is ``partial_kernel``'s."""
     monkeypatch.setenv("L20_PD_FUSED", "0")
     monkeypatch.setenv("L20_PD_FUSED_SPLIT", "0")
+
+
+def pytest_generate_tests(metafunc):
+    """A module's PARTIAL_KERNELS ("persistent", "units") runs each of its tests once per
+    kernel; without one the library chooses."""
+    kernels = getattr(metafunc.module, "PARTIAL_KERNELS", None)
+    if kernels:
+        metafunc.parametrize("partial_kernel", kernels, indirect=True)
+
+
+@pytest.fixture(autouse=True)
+def partial_kernel(request, monkeypatch):
+    """The partial kernel of split calls: the persistent work queue or pd_units, where the
+    shape allows it (at most 256 sequences)."""
+    kernel = getattr(request, "param", None)
+    if kernel:
+        monkeypatch.setenv("L20_PD_UNITS", {"persistent": "0", "units": "1"}[kernel])
+    return kernel

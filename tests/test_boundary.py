@@ -277,6 +277,8 @@ def test_partial_kernel_rule(monkeypatch):
     assert cabi.partial_kernel(a) == "pd_fp8_partial"
     monkeypatch.setenv("L20_PD_UNITS", "1")
     assert cabi.partial_kernel(a) == "pd_units"
+    monkeypatch.setenv("L20_PD_FUSED_SPLIT", "0")  # the split mode's alone
+    assert cabi.partial_kernel(a) == "pd_units"
     monkeypatch.setenv("L20_PD_UNITS", "0")
     a.batch = 17
     assert cabi.partial_kernel(a) == "pd_fp8_partial"

@@ -71,6 +71,7 @@ def test_oracle_reproduces_golden(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("partial_kernel", ["persistent", "units"], indirect=True)
 @pytest.mark.parametrize("name,split", GPU_CASES)
 def test_hip_op_matches_golden(name, split):
     if not torch.cuda.is_available():

@@ -32,6 +32,7 @@ import torch
 import pd_helpers as H
 
 pytestmark = pytest.mark.gpu
+PARTIAL_KERNELS = ["persistent", "units"]
 
 L = 32768          # one long sequence: 2048 pages, 32 to 64 splits
 HQ, HKV, D = 8, 1, 128

@@ -17,6 +17,7 @@ import torch
 import pd_helpers as H
 
 pytestmark = pytest.mark.gpu
+PARTIAL_KERNELS = ["persistent", "units"]
 
 N_CASES = 120
 N_E5M2 = 24
@@ -99,7 +100,7 @@ N_SPLIT_MODE = 48
 def test_random_shape_split_mode(case, monkeypatch):
     """A third seed range with the single-launch kernel's split mode forced
     (L20_PD_FUSED_SPLIT=1) at the splits it accepts (256, 512, 1024 tokens);
-    calls with one split slot still run the persistent kernel."""
+    calls with one split slot run the partial kernel of `partial_kernel`."""
     monkeypatch.setenv("L20_PD_FUSED_SPLIT", "1")
     c = draw(case, seed_base=9000)
     c["split"] = int(np.random.default_rng(9000 + case).choice([256, 256, 512, 1024]))

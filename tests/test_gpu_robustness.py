@@ -27,6 +27,7 @@ import torch
 import pd_helpers as H
 
 pytestmark = pytest.mark.gpu
+PARTIAL_KERNELS = ["persistent"]
 
 
 def _call_args(inp, split, out, lse):

@@ -13,6 +13,7 @@ import torch
 import pd_helpers as H
 
 pytestmark = pytest.mark.gpu
+PARTIAL_KERNELS = ["persistent", "units"]
 
 
 def random_tree(s, rng):

@@ -2,9 +2,12 @@
 the chip (GPU), forced with L20_PD_UNITS=1: output and LSE against the oracle at
 the shapes where its schedule can go wrong -- units shared by 8, 4, 2 and 1 waves
 (fewer units than waves, parts without blocks), several units per wave (the grid
-capped), lanes holding one and several sequences, empty and one-token rows, splits
-that are not whole blocks, odd head counts, every cache type, page size and page
-list, draft rows and trees over one and two query tiles -- and the library's choice.
+capped), each with every cache type, pages of 16, 32 and 64 tokens, block tables and
+page lists, draft rows and trees over one and two query tiles; lanes holding one and
+several sequences, empty and one-token rows, splits that are not whole blocks, odd
+head counts -- and the library's choice.  The entry points above it (tree
+verification, the hook functions, strided caches, two streams, the allocation-free
+entry) run on it in their own tests (PARTIAL_KERNELS).
 """
 
 import zlib
@@ -25,7 +28,7 @@ PDT = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}
 @pytest.fixture(autouse=True)
 def _units(monkeypatch):
     monkeypatch.setenv("L20_PD_FUSED", "0")
-    monkeypatch.setenv("L20_PD_FUSED_SPLIT", "2")  # neither the split mode nor the persistent kernel
+    monkeypatch.setenv("L20_PD_FUSED_SPLIT", "0")
     monkeypatch.setenv("L20_PD_UNITS", "1")
 
 
@@ -53,9 +56,9 @@ def _run(inp, split, pdt, kernels, kernel="pd_units"):
 
 CASES = [
     # name, batch, hq, hkv, d, lens, q_len, per_head, fp8, page, split, pdt, workgroups (0: the CUs)
-    ("p8_one_unit", 1, 8, 1, 128, [400], 1, False, "e4m3fn", 16, 512, "fp32", 0),
-    ("p8_empty_parts", 2, 8, 2, 128, [1, 90], 1, True, "e4m3fn", 16, 512, "fp32", 0),
-    ("p2_p4", 5, 28, 4, 128, [1, 15, 1025, 2048, 600], 1, True, "e4m3fn", 16, 512, "fp16", 12),
+    ("one_unit", 1, 8, 1, 128, [400], 1, False, "e4m3fn", 16, 512, "fp32", 0),
+    ("empty_parts", 2, 8, 2, 128, [1, 90], 1, True, "e4m3fn", 16, 512, "fp32", 0),
+    ("ragged_fp16", 5, 28, 4, 128, [1, 15, 1025, 2048, 600], 1, True, "e4m3fn", 16, 512, "fp16", 12),
     ("many_per_wave", 7, 16, 2, 128, [700, 1, 0, 64, 1300, 90, 513], 1, True, "e4m3fn", 16, 64, "fp32", 1),
     ("two_workgroups", 9, 12, 3, 128, [333, 5, 800, 64, 65, 0, 1, 1100, 127], 1, False, "e4m3fn", 16, 128, "bf16", 2),
     ("split80", 4, 8, 2, 128, [900, 81, 80, 79], 1, False, "e4m3fn", 16, 80, "fp32", 3),
@@ -77,6 +80,63 @@ def test_units_match_oracle(case, monkeypatch, kernels):
                            seed=zlib.crc32(name.encode()) % 1000, garbage_tail=True)
     out, lse = _run(inp, split, PDT[pdt], kernels)
     H.compare(out, lse, *H.run_oracle(inp))
+
+
+def _unit_count(lens, split, hkv):
+    return hkv * sum(max(1, -(-x // split)) for x in lens)
+
+
+def _groups(units, waves, tiles):
+    """The smallest grid on which `waves` waves share a unit (at most half of the chip's
+    waves with one query tile, all of them with two); 0: one workgroup for all units."""
+    fill = 4 if tiles == 1 else 8
+    return -(-units * waves // fill) if waves else 1
+
+
+SHARED = [
+    # name, hq, hkv, d, q_len, tree, cache, page, csr
+    ("fp8", 8, 2, 128, 1, False, "e4m3fn", 16, False),
+    ("fp8_d64", 8, 2, 64, 1, False, "e4m3fn", 32, False),
+    ("e5m2_verify", 8, 2, 128, 4, False, "e5m2", 16, False),
+    ("fp8_tree", 8, 2, 128, 4, True, "e4m3fn", 16, False),
+    ("fp8_tree_2tiles", 16, 2, 128, 4, True, "e4m3fn", 16, False),
+    ("fp8_tree_18cols", 12, 2, 128, 3, True, "e4m3fn", 64, False),
+    ("e5m2_tree_2tiles_d64", 16, 2, 64, 4, True, "e5m2", 16, False),
+    ("fp8_verify_2tiles_d64", 16, 2, 64, 4, False, "e4m3fn", 16, False),
+    ("bf16", 8, 2, 128, 1, False, "bf16", 16, False),
+    ("bf16_csr_pages32", 8, 2, 128, 1, False, "bf16", 32, True),
+    ("fp16_tree_d64", 8, 2, 64, 4, True, "fp16", 64, False),
+    ("bf16_tree_2tiles", 16, 2, 128, 4, True, "bf16", 16, False),
+    ("fp16_tree_2tiles_csr", 16, 2, 128, 4, True, "fp16", 16, True),
+    ("fp16_tree_18cols_d64", 12, 2, 64, 3, True, "fp16", 32, False),
+    ("bf16_verify_2tiles_d64", 16, 2, 64, 4, False, "bf16", 64, False),
+]
+
+
+@pytest.mark.parametrize("waves", [8, 4, 2, 1, 0])
+@pytest.mark.parametrize("case", SHARED, ids=[c[0] for c in SHARED])
+def test_units_shared_by_waves(case, waves, monkeypatch):
+    """Every kind of call with 8, 4, 2 and 1 waves to a unit, and all units in one
+    workgroup; ragged, so that the longest sequence's splits outnumber the others'."""
+    name, hq, hkv, d, q_len, tree, cache, page, csr = case
+    lens, split = [2000, 30, 545, 8, 64, 7], 512
+    tiles = (hq // hkv * q_len + 15) // 16
+    monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", str(_groups(_unit_count(lens, split, hkv), waves, tiles)))
+    seed = zlib.crc32(name.encode()) % 1000
+    fp8 = cache in ("e4m3fn", "e5m2")
+    if fp8:
+        inp = H.make_synthetic(len(lens), hq, hkv, d, lens, q_len=q_len, per_head=True, fp8=cache, page=page,
+                               seed=seed, garbage_tail=True)
+    else:
+        inp = H.make_synthetic16(len(lens), hq, hkv, d, lens, dtype=torch.float16 if cache == "fp16" else torch.bfloat16,
+                                 q_len=q_len, page=page, seed=seed, garbage_tail=True, csr_pad=1)
+    if tree:
+        w = np.random.default_rng(seed).integers(0, 2**32, size=(len(lens), q_len), dtype=np.int64)
+        inp["tree_mask"] = torch.from_numpy(np.where(w >= 2**31, w - 2**32, w).astype(np.int32)).cuda()
+    if fp8:
+        H.compare(*H.run_op(inp, split), *H.run_oracle(inp))
+    else:
+        H.compare(*H.run_op16(inp, split, csr=csr), *H.run_oracle16(inp, csr=csr))
 
 
 @pytest.mark.parametrize("batch", [65, 256])

@@ -13,6 +13,7 @@ import torch
 import pd_helpers as H
 
 pytestmark = pytest.mark.gpu
+PARTIAL_KERNELS = ["persistent", "units"]
 FIXTURE = Path(__file__).parent / "fixtures" / "vllm_rocm"
 
 

@@ -8,6 +8,7 @@ import torch
 import pd_helpers as H
 
 pytestmark = pytest.mark.gpu
+PARTIAL_KERNELS = ["persistent", "units"]
 
 
 @pytest.fixture(scope="module", autouse=True)
