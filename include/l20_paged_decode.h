@@ -231,6 +231,11 @@ int32_t l20_pd_single_launch(const l20_pd_fp8_args *args);
  * units per CU and head_dim 64 beyond 32 (batch x num_kv_heads x splits). */
 int32_t l20_pd_partial_kernel(const l20_pd_fp8_args *args);
 
+/* Launches of the persistent partial kernel by this process so far: the calls
+ * that took a work-queue slot (no other path has a queue).  A test hook with no
+ * reference counterpart. */
+uint32_t l20_pd_queue_launches(void);
+
 /* Sets every work-queue counter of the current device to `value` (after a
  * device synchronize), as a launch that gave up mid-way or shared a slot with
  * another leaves it.  A test hook with no reference counterpart: with a value

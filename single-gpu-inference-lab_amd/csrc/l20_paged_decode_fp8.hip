@@ -3325,9 +3325,6 @@ int32_t run(const l20_pd_fp8_args *a, void *stream_ptr, int stages, int kinds) {
   const int group = a->num_q_heads / a->num_kv_heads;
   const int nqt = (group * a->q_len + 15) / 16;
   l20pd::PartialParams pp = partial_params(*a, n_s);
-  pp.queue_slot = counter_slot(stream);
-  pp.spin_cap = spin_limit();
-  pp.launch_tag = g_launch_seq.fetch_add(1u, std::memory_order_relaxed);
   const l20pd::MergeParams mp = merge_params(*a, pp.num_splits);
   const bool bf16 = a->query_dtype == L20_PD_BF16;
   const int rows = a->batch * a->q_len;
@@ -3366,6 +3363,11 @@ int32_t run(const l20_pd_fp8_args *a, void *stream_ptr, int stages, int kinds) {
     else
       e = bf16 ? launch_units<__bf16, 0>(pp, D, nqt, units, stream) : launch_units<_Float16, 0>(pp, D, nqt, units, stream);
   } else if (stages & kPartial) {
+    // Only the persistent kernel has a work queue: a call on another path must not
+    // take a slot (and with it evict another stream's, or a captured launch's).
+    pp.queue_slot = counter_slot(stream);
+    pp.spin_cap = spin_limit();
+    pp.launch_tag = g_launch_seq.fetch_add(1u, std::memory_order_relaxed);
     const int D = a->head_dim, B = a->batch, H = a->num_kv_heads;
     if (kv16)
       e = bf16 ? launch_partial_shape<__bf16, 1>(pp, D, nqt, B, H, stream)
@@ -3529,6 +3531,8 @@ int32_t l20_pd_partial_kernel(const l20_pd_fp8_args *a) {
   if (fused_split_fits(*a, pp, nqt, kv16)) return 2;
   return units_fit(*a, pp, nqt, kv16) ? 3 : 0;
 }
+
+uint32_t l20_pd_queue_launches(void) { return g_launch_seq.load(std::memory_order_relaxed); }
 
 int32_t l20_pd_set_queue_counters(uint64_t value) {
   g_last_error[0] = '\0';

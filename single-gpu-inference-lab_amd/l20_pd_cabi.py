@@ -32,6 +32,7 @@ EXPORTED = (
     "l20_pd_device_errors",
     "l20_pd_set_spin_limit",
     "l20_pd_set_queue_counters",
+    "l20_pd_queue_launches",
     "l20_pd_single_launch",
     "l20_pd_partial_kernel",
     "l20_pd_split_out",
@@ -145,6 +146,8 @@ def load(path: Optional[Path] = None) -> ctypes.CDLL:
     lib.l20_pd_set_spin_limit.restype = _i32
     lib.l20_pd_set_queue_counters.argtypes = [ctypes.c_uint64]
     lib.l20_pd_set_queue_counters.restype = _i32
+    lib.l20_pd_queue_launches.argtypes = []
+    lib.l20_pd_queue_launches.restype = ctypes.c_uint32
     for name in ("l20_pd_single_launch", "l20_pd_partial_kernel"):
         getattr(lib, name).argtypes = [args_p]
         getattr(lib, name).restype = _i32
@@ -349,6 +352,12 @@ def set_queue_counters(value: int, lib: Optional[ctypes.CDLL] = None) -> None:
     lib = lib or load()
     if lib.l20_pd_set_queue_counters(int(value)) != L20_PD_OK:
         raise RuntimeError(last_error(lib))
+
+
+def queue_launches(lib: Optional[ctypes.CDLL] = None) -> int:
+    """``l20_pd_queue_launches``: this process's launches of the persistent partial
+    kernel, the only ones that take a work-queue slot (a test hook)."""
+    return int((lib or load()).l20_pd_queue_launches())
 
 
 def check(args: L20PdFp8Args, lib: Optional[ctypes.CDLL] = None) -> None:

@@ -33,6 +33,16 @@ def _units(monkeypatch):
 
 
 @pytest.fixture
+def no_queue():
+    """The persistent kernel did not run: no call took a work-queue slot."""
+    import l20_pd_cabi as cabi
+
+    before = cabi.queue_launches()
+    yield
+    assert cabi.queue_launches() == before
+
+
+@pytest.fixture
 def kernels(monkeypatch):
     """The partial kernel of every call made through the C ABI, as the library names it."""
     import l20_pd_cabi as cabi
@@ -115,7 +125,7 @@ SHARED = [
 
 @pytest.mark.parametrize("waves", [8, 4, 2, 1, 0])
 @pytest.mark.parametrize("case", SHARED, ids=[c[0] for c in SHARED])
-def test_units_shared_by_waves(case, waves, monkeypatch):
+def test_units_shared_by_waves(case, waves, monkeypatch, no_queue):
     """Every kind of call with 8, 4, 2 and 1 waves to a unit, and all units in one
     workgroup; ragged, so that the longest sequence's splits outnumber the others'."""
     name, hq, hkv, d, q_len, tree, cache, page, csr = case
@@ -152,7 +162,7 @@ def test_units_many_sequences(batch, monkeypatch, kernels):
 
 @pytest.mark.parametrize("groups", ["1", "5", "256"])
 @pytest.mark.parametrize("case", range(32))
-def test_units_random_shape(case, groups, monkeypatch):
+def test_units_random_shape(case, groups, monkeypatch, no_queue):
     monkeypatch.setenv("L20_PD_MAX_WORKGROUPS", groups)
     c = draw(case, seed_base=13000)
     print(case, c, flush=True)
@@ -201,3 +211,42 @@ def test_library_takes_the_units_kernel(monkeypatch, kernels):
     big = H.make_synthetic(257, 4, 2, 64, [1 + 7 * (i % 90) for i in range(257)], seed=4)
     out, lse = _run(big, 64, torch.float32, kernels, kernel="pd_fp8_partial")
     H.compare(out, lse, *H.run_oracle(big))
+
+
+def test_only_the_persistent_kernel_takes_a_queue_slot(monkeypatch):
+    """Eager and captured calls of every path: a slot (16 for captured calls) goes to
+    launches that have a work queue and to no other."""
+    import l20_pd_cabi as cabi
+
+    inp = H.make_synthetic(6, 28, 4, 128, [900, 31, 1000, 0, 512, 77], seed=5)
+    exp = H.run_oracle(inp)
+    q = inp["query"]
+    work = H.workspace(inp, 256)
+    out = torch.empty_like(q)
+    ks, _ = H._scales(inp["k_scale"])
+    vs, _ = H._scales(inp["v_scale"])
+
+    def call():
+        torch.ops.l20_stack.paged_decode_fp8_e4m3_split_out(
+            q, inp["key_cache"], inp["value_cache"], inp["block_table"], inp["seq_lens"], *work, out, ks, vs,
+            inp["max_seq_len"], 256, inp["softmax_scale"], None, None)
+
+    for env, slots in (({"L20_PD_UNITS": "1"}, 0), ({"L20_PD_FUSED": "1"}, 0), ({"L20_PD_FUSED_SPLIT": "1"}, 0),
+                       ({"L20_PD_UNITS": "0"}, 1)):
+        with monkeypatch.context() as m:
+            for name, value in env.items():
+                m.setenv(name, value)
+            before = cabi.queue_launches()
+            call()
+            assert cabi.queue_launches() == before + slots
+            torch.cuda.synchronize()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                call()
+            assert cabi.queue_launches() == before + 2 * slots
+        for _ in range(3):
+            out.zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            H.compare(out, None, *exp, check_lse=False)
+        assert cabi.queue_launches() == before + 2 * slots
