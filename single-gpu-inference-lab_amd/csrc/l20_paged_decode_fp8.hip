@@ -2030,8 +2030,11 @@ __global__ __launch_bounds__(64 * kFusedWaves) void pd_fp8_fused(PartialParams p
 // KV heads 31.1 -> 13.9; 8 x 4096 33.2 -> 19.8; 16 x 4096 35.7 -> 28.3; 48 x 4096
 // 76.9 -> 69.5; 128 x uniform 100-4096 108.3 -> 99.8; 32 lognormal sequences to
 // 8192, 4 KV heads, bf16 caches 63.7 -> 27.7; verification (32 x uniform to 3000,
-// 8 drafts) 51.0 -> 33.0; 128 lognormal sequences, 4 KV heads 45.7 -> 45.8; 100 x
-// 2048, 2 KV heads 25.1 -> 27.2 (the worst found).
+// 8 drafts) 51.0 -> 33.0; 128 lognormal sequences, 4 KV heads 45.7 -> 45.8.
+// It loses on equal lengths where some workgroups take a unit more than the others:
+// 100 x 2048 tokens, 2 KV heads (3.1 units per CU) 25.7 -> 27.2; 100 x 2048, 8 KV heads
+// (12.5) 80.8 -> 84.7, where 96 of them (12.0) take 81.8 -> 73.2.  units_fit has the
+// other side.
 //
 // Block stream: NB blocks in flight across unit boundaries, as in the persistent
 // kernel.  A cursor runs NB blocks ahead of the computed block; the entries of the
@@ -3023,8 +3026,12 @@ hipError_t launch_units_tiles(l20pd::PartialParams pp, int head_dim, int64_t uni
   pp.heads_recip = recip32(pp.num_kv_heads);
   pp.split_recip = recip32(pp.split_size);
   // Blocks in flight per wave: two; one with two query tiles of fp8 caches (two
-  // would spill) and, as in the persistent kernel, for fp8 splits of 1024 tokens
-  // (2 x 131072 tokens, 8 KV heads 89.3 -> 87.4 us per call, 3 x 60000 69.3 -> 63.8).
+  // would spill) and, as in the persistent kernel, for fp8 splits of 1024 tokens, where
+  // one is ahead with 5 to 8 units per CU of equal lengths (us per call with one and two,
+  // 8 KV heads: 2 x 131072 tokens 87.4, 89.3; 3 x 60000 68.7, 74.3; 24 x 9000 79.1, 82.2)
+  // and two elsewhere (8 x 16000 52.0, 49.9, uniform to 16000 47.3, 36.9; 3 x 60000, 4 KV
+  // heads 48.8, 38.7).  Neither is behind the persistent kernel by more than 2% (57.9,
+  // 52.3 and 48.2 for the last three).
   constexpr int NB = (NQT == 1 || KT == 1) ? 2 : 1;
   if constexpr (KT != 1 && NQT == 1)
     if (head_dim == 128 && pp.split_size >= 1024) {
@@ -3050,7 +3057,13 @@ hipError_t launch_units(const l20pd::PartialParams &pp, int head_dim, int nqt, i
 // the host can see): 128 lognormal sequences, 4 KV heads 81.8 against 83.2 us per
 // call (8192 units at most), 64 of them 45.8 against 44.4 (4096).  At head_dim 64,
 // beyond 32: 200 x uniform to 3000, 8 KV heads 88.4 against 91.0 (9600), 100 of
-// them 53.6 against 46.5 (4800).  L20_PD_UNITS=0/1 overrides the size rule (tests and
+// them 53.6 against 46.5 (4800).  Within the bounds equal lengths can be faster on the
+// persistent kernel, but the host cannot tell them from ragged ones, which gain more
+// (512-token splits, us per call on the persistent kernel and here, equal lengths,
+// uniform from an eighth, lognormal): 100 sequences to 2048 tokens, 2 KV heads 25.7 27.1,
+// 24.6 23.4, 23.8 17.0; 8 KV heads 83.5 85.7, 54.1 54.0, 36.3 31.2; 8 KV heads of 64
+// 61.5 66.4, 40.2 41.4, 31.4 25.5; 24 to 9000, 1024-token splits, 8 KV heads of 64
+// 57.0 62.1, 49.7 34.6, 45.9 22.9.  L20_PD_UNITS=0/1 overrides the size rule (tests and
 // measurement).
 bool units_fit(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, int nqt, bool kv16) {
   if (nqt > 2 || a.batch > l20pd::kUnitMaxBatch) return false;

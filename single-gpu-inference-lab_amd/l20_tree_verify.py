@@ -96,11 +96,16 @@ def _tree_split_size(entries: int, num_kv_heads: int, columns: int, max_len: int
     calls of more than 16 query columns take at least 512 tokens once that leaves more
     units (entry, split, KV head) than the GPU has CUs, and 1024 once that leaves four
     times as many.  Every such unit writes 32 fp32 rows (16 KB at head_dim 128), which
-    at the library's 128 or 256 tokens cost more than the finer splits give (us per
-    call at 128, 256, 512, 1024 tokens; 32 / 8 heads, 8 drafts: 16 x 500-3000 tokens
-    37.0, 34.9, 33.8, 35.9; 64 x 500-2000 83.6, 68.3, 56.9, 54.5; 24 drafts beside 4 x
-    3999 bf16 tokens 84.8, 66.3, 61.1, 64.7; with 8 columns, 16 x 500-3000 20.5, 18.9,
-    19.9, 25.0)."""
+    at the library's 64 to 256 tokens cost more than the finer splits give.  us per
+    call at 256, 512 and 1024 tokens, 32 / 8 heads, 8 drafts: 16 x 500-3000 tokens 34.3,
+    33.2, 36.3; 64 x 333-2000 67.9, 57.4, 55.2 (78.0 at the library's 128); 24 drafts
+    beside 4 x 3999 bf16 tokens 63.6, 58.2, 62.1.  Of 126 calls that the rule changes
+    (head_dim 64 and 128, 1 to 8 KV heads, fp8 and bf16 caches, 3 to 200 sequences, 400
+    to 3200 units of 512 tokens) four are slower by it, all of 24 x 333-2000 tokens, 8 KV
+    heads (256 tokens are 2-9% better); the others take 1.0 to 3.3 times as long at the
+    library's split.  From 2400 units 512 can beat 1024 (100 x 250-1500: 61.9, 80.8);
+    below the first line, 16 bf16 prefixes of 1000 tokens with 16 drafts of 16 / 2 heads
+    (256 units) would take 33.5 at 512, and take 45.2 at the library's 64."""
     split = default_split_size(entries, num_kv_heads, max_len, device)
     if columns > 16:
         cus = gpu_cus(device)
