@@ -722,21 +722,31 @@ void launch_fast_rows(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uin
     hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
 }
 
-// Rows per lane.  A call is a chain of dependent loads, so what decides is whether
-// its workgroups are on the chip at once: 8 a CU of one row per lane (2048), 6 of
-// two (1536, the rows of 3072 of one).  Up to 2048 workgroups one row, up to 3072
-// two, beyond them one again (the shorter last round), until the stream is long
-// enough for the loads in flight to count: 16384 with fp8 caches, whose quantiser
-// needs the waves, 4096 with 16-bit ones.  us per call with one and two rows, in a
-// graph, by workgroups of one row, 28 + 4 heads of 128 with an fp8 and a bf16 cache:
-// 1024 4.2, 5.0 and 3.8, 4.2; 1900 5.2, 6.0 and 5.5, 5.6; 2100 7.0, 6.5 and 6.5, 6.2;
-// 2800 7.9, 7.3 and 7.5, 7.3; 3300 8.5, 10.1 and 8.4, 9.5; 4000 10.1, 11.0 and 10.1,
-// 10.4; 7000 16.7, 17.7 and 16.7, 16.4; 16000 33.6, 34.7 and 34.1, 34.0; 32000 63.4,
-// 63.1 and 63.0, 63.6.  8 + 1 heads, bf16 cache: 9216 22.0, 21.1.
+// Rows per lane, by `one`, the workgroups of one row per lane.  A call is a chain of
+// dependent loads, so what decides is whether its workgroups are on the chip at once:
+// 8 a CU of one row per lane (2048), 6 of two (1536, the rows of 3072 of one; 5 with
+// fp8 caches and fp32 tables, whose words take twice the registers).  Up to 2048 one
+// row, up to 3072 two, beyond them one again (the shorter last round), until the
+// stream is long enough for the loads in flight to count: 20480 with fp8 caches, whose
+// quantiser needs the waves, 4096 with 16-bit ones, never with fp32 tables.  us per
+// call with one and two rows, in a graph, by `one`, 28 + 4 heads of 128 with an fp8 and
+// a bf16 cache, 16-bit tables: 1024 4.2, 5.0 and 3.8, 4.2; 1900 5.2, 6.0 and 5.5, 5.6;
+// 2100 7.0, 6.5 and 6.5, 6.2; 2800 7.9, 7.3 and 7.5, 7.3; 3300 8.5, 10.1 and 8.4, 9.5;
+// 4000 10.1, 11.0 and 10.1, 10.4; 7000 16.7, 17.7 and 16.7, 16.4; 16000 33.6, 34.7 and
+// 34.1, 34.0; 18000 37.6, 38.5 and 37.9, 38.1; 25500 51.3, 51.1 and 51.0, 51.9; 32000
+// 63.4, 63.1 and 63.0, 63.6.  8 + 1 heads, bf16 cache: 9216 22.0, 21.1.  32 + 8 heads,
+// fp32 tables: 2100 7.5, 7.8 and 7.0, 7.4; 2500 9.2, 8.4 and 8.5, 8.2; 3000 9.9, 10.9
+// and 9.6, 9.1; 3200 10.4, 11.4 and 9.8, 10.1; 9000 21.3, 24.2 and 22.0, 24.3; 16000
+// 34.6, 38.0 and 34.7, 38.0; 32768 66.0, 73.4 and 65.2, 68.5.
+int rows_per_lane(int64_t one, bool fp8_cache, bool fp32_table) {
+  if (one <= 2048) return 1;
+  if (one <= (fp8_cache && fp32_table ? 2560 : 3072)) return 2;
+  return fp32_table || one <= (fp8_cache ? 20480 : 4096) ? 1 : 2;
+}
 template <typename T, int CT>
 void launch_fast(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uint32_t rows_all, hipStream_t s) {
   const int64_t one = ((int64_t)rows_all + 4 * (64 / (p.d / 8)) - 1) / (4 * (64 / (p.d / 8)));
-  if (one <= 2048 || (one > 3072 && one <= (CT == 0 ? 16384 : 4096))) launch_fast_rows<T, CT, 1>(p, cs_dtype, rows_q, rows_all, s);
+  if (rows_per_lane(one, CT == 0, cs_dtype == 2) == 1) launch_fast_rows<T, CT, 1>(p, cs_dtype, rows_q, rows_all, s);
   else launch_fast_rows<T, CT, 2>(p, cs_dtype, rows_q, rows_all, s);
 }
 

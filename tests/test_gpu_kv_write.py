@@ -245,15 +245,19 @@ def test_fp8_scales_match_oracle(per_head):
 
 
 @pytest.mark.parametrize("fp8", [True, False], ids=["fp8", "bf16"])
-@pytest.mark.parametrize("tokens", [1, 1023, 1025, 1536, 1537, 2048, 2049, 2731, 8192, 8193])
-def test_one_and_two_rows_per_lane(tokens, fp8):
+@pytest.mark.parametrize("tokens,table", [(t, "bf16") for t in (1, 1023, 1025, 1536, 1537, 2048, 2049, 2731, 8192,
+                                                                8193, 10240, 10241)]
+                         + [(t, "fp32") for t in (1025, 1280, 1281, 1537, 2049, 10241)])
+def test_one_and_two_rows_per_lane(tokens, table, fp8):
     """Both sides of each line of the rows-per-lane rule (2048, 3072 and, by the cache type,
-    4096 or 16384 workgroups: 1024, 1536, 2048 and 8192 tokens of 32 head rows of 128), the
-    last workgroup full and not: bit exact against the producer's oracle."""
+    4096 or 20480 workgroups: 1024, 1536, 2048 and 10240 tokens of 32 head rows of 128; with
+    fp32 tables 2048 and, by the cache type, 2560 or 3072), the last workgroup full and not:
+    bit exact against the producer's oracle."""
     from oracle import kv_write_ref as kw
     import l20_rope_kv
 
-    c = _case(max(tokens, 2), 28, 4, 128, 128, torch.bfloat16, torch.bfloat16, seed=tokens)
+    cs_dtype = torch.float32 if table == "fp32" else torch.bfloat16
+    c = _case(max(tokens, 2), 28, 4, 128, 128, torch.bfloat16, cs_dtype, seed=tokens)
     c = {k: (v[:tokens] if isinstance(v, torch.Tensor) and k != "cs" else v) for k, v in c.items()}
     q, k = c["q"].cuda(), c["k"].cuda()
     kc = torch.zeros(c["pages"], 16, 4, 128, dtype=torch.float8_e4m3fn if fp8 else torch.bfloat16).cuda()
