@@ -266,7 +266,11 @@ __device__ __forceinline__ int quant4(const float (&x)[4], float scale) {
 // Rows [0, rows_q) are Q head rows (token r / Hq, head r % Hq), the next
 // rows_k are K head rows (token r / Hkv): rotated in place, and for K also the
 // K and V cache writes.  Four waves; a lane group of lpr = D/8 lanes per row.
-template <typename T, int CT, int CS, int ROWS>
+// POS_FIRST: the positions load ahead of the rows, so that the cos/sin loads wait for
+// them alone.  Only for two rows on long streams (launch_fast): 16384 tokens of 28 + 4
+// heads, fp8 and bf16 caches, 63.6 -> 62.7 and 63.3 -> 62.5 us; 1050 tokens would go
+// from 6.8 to 7.7, and one row gains nothing (4.56, 4.64 at 500).
+template <typename T, int CT, int CS, int ROWS, bool POS_FIRST>
 __global__ __launch_bounds__(256) void kv_rope_write8(Params p, uint32_t rows_q, uint32_t rows_all) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
@@ -287,37 +291,68 @@ __global__ __launch_bounds__(256) void kv_rope_write8(Params p, uint32_t rows_q,
   T *row[ROWS];
   int head[ROWS];
   bool live[ROWS], is_k[ROWS];
+  if constexpr (POS_FIRST) {
+    int64_t tok[ROWS];
 #pragma unroll
-  for (int u = 0; u < ROWS; ++u) {
-    const uint32_t r = first + (uint32_t)((u * 4 + wave) * rpw + g);
-    live[u] = g < rpw && r < rows_all;
-    is_k[u] = r >= rows_q;
-    int64_t t = 0;
-    int h = 0;
-    if (live[u]) {
-      if (!is_k[u]) {
-        const uint32_t q = r / (uint32_t)p.hq;
-        t = q;
-        h = (int)(r - q * (uint32_t)p.hq);
-        row[u] = reinterpret_cast<T *>(p.q) + t * p.q_st + (int64_t)h * p.q_sh;
-      } else {
-        const uint32_t rk = r - rows_q;
-        const uint32_t q = rk / (uint32_t)p.hkv;
-        t = q;
-        h = (int)(rk - q * (uint32_t)p.hkv);
-        row[u] = reinterpret_cast<T *>(p.k) + t * p.k_st + (int64_t)h * p.k_sh;
-        vw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(reinterpret_cast<const T *>(p.v) + t * p.v_st +
-                                                 (int64_t)h * p.v_sh + e0));
-        slot[u] = p.slots[t];
+    for (int u = 0; u < ROWS; ++u) {
+      const uint32_t r = first + (uint32_t)((u * 4 + wave) * rpw + g);
+      live[u] = g < rpw && r < rows_all;
+      is_k[u] = r >= rows_q;
+      const uint32_t n = is_k[u] ? r - rows_q : r, heads = (uint32_t)(is_k[u] ? p.hkv : p.hq);
+      tok[u] = n / heads;
+      head[u] = (int)(n % heads);
+      pos[u] = 0;
+      if (live[u] && rot_lane) pos[u] = p.pos[tok[u]];
+    }
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      row[u] = is_k[u] ? reinterpret_cast<T *>(p.k) + tok[u] * p.k_st + (int64_t)head[u] * p.k_sh
+                       : reinterpret_cast<T *>(p.q) + tok[u] * p.q_st + (int64_t)head[u] * p.q_sh;
+      if (!live[u]) continue;
+      xw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(row[u] + e0));
+      if (is_k[u]) {
+        vw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(
+            reinterpret_cast<const T *>(p.v) + tok[u] * p.v_st + (int64_t)head[u] * p.v_sh + e0));
+        slot[u] = p.slots[tok[u]];
         if constexpr (CT == 0) {
-          ksc[u] = p.k_scale_ph ? p.k_scale_ph[h] : p.k_scale;
-          vsc[u] = p.v_scale_ph ? p.v_scale_ph[h] : p.v_scale;
+          ksc[u] = p.k_scale_ph ? p.k_scale_ph[head[u]] : p.k_scale;
+          vsc[u] = p.v_scale_ph ? p.v_scale_ph[head[u]] : p.v_scale;
         }
       }
-      xw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(row[u] + e0));
-      pos[u] = p.pos[t];
     }
-    head[u] = h;
+  } else {
+#pragma unroll
+    for (int u = 0; u < ROWS; ++u) {
+      const uint32_t r = first + (uint32_t)((u * 4 + wave) * rpw + g);
+      live[u] = g < rpw && r < rows_all;
+      is_k[u] = r >= rows_q;
+      int64_t t = 0;
+      int h = 0;
+      if (live[u]) {
+        if (!is_k[u]) {
+          const uint32_t q = r / (uint32_t)p.hq;
+          t = q;
+          h = (int)(r - q * (uint32_t)p.hq);
+          row[u] = reinterpret_cast<T *>(p.q) + t * p.q_st + (int64_t)h * p.q_sh;
+        } else {
+          const uint32_t rk = r - rows_q;
+          const uint32_t q = rk / (uint32_t)p.hkv;
+          t = q;
+          h = (int)(rk - q * (uint32_t)p.hkv);
+          row[u] = reinterpret_cast<T *>(p.k) + t * p.k_st + (int64_t)h * p.k_sh;
+          vw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(reinterpret_cast<const T *>(p.v) + t * p.v_st +
+                                                   (int64_t)h * p.v_sh + e0));
+          slot[u] = p.slots[t];
+          if constexpr (CT == 0) {
+            ksc[u] = p.k_scale_ph ? p.k_scale_ph[h] : p.k_scale;
+            vsc[u] = p.v_scale_ph ? p.v_scale_ph[h] : p.v_scale;
+          }
+        }
+        xw[u] = __builtin_nontemporal_load(reinterpret_cast<const i32x4 *>(row[u] + e0));
+        pos[u] = p.pos[t];
+      }
+      head[u] = h;
+    }
   }
   // ---- cos / sin of the lanes' dims ----
   CosSin<CS> cs[ROWS];
@@ -710,16 +745,19 @@ bool fast_path_ok(const l20_pd_kv_write_args &a) {
   return true;
 }
 
-template <typename T, int CT, int ROWS>
+template <typename T, int CT, int ROWS, bool POS_FIRST>
 void launch_fast_rows(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uint32_t rows_all, hipStream_t s) {
   const int64_t rows_per_wg = (int64_t)4 * (64 / (p.d / 8)) * ROWS;
   const dim3 grid((unsigned)((rows_all + rows_per_wg - 1) / rows_per_wg));
-  if (cs_dtype == 2)
-    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 2, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
-  else if (cs_dtype == 1)
-    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 1, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+  if constexpr (!POS_FIRST)  // never with fp32 tables (rows_per_lane)
+    if (cs_dtype == 2) {
+      hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 2, ROWS, false>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+      return;
+    }
+  if (cs_dtype == 1)
+    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 1, ROWS, POS_FIRST>), grid, dim3(256), 0, s, p, rows_q, rows_all);
   else
-    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0, ROWS>), grid, dim3(256), 0, s, p, rows_q, rows_all);
+    hipLaunchKernelGGL((l20kv::kv_rope_write8<T, CT, 0, ROWS, POS_FIRST>), grid, dim3(256), 0, s, p, rows_q, rows_all);
 }
 
 // Rows per lane, by `one`, the workgroups of one row per lane.  A call is a chain of
@@ -732,12 +770,12 @@ void launch_fast_rows(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uin
 // call with one and two rows, in a graph, by `one`, 28 + 4 heads of 128 with an fp8 and
 // a bf16 cache, 16-bit tables: 1024 4.2, 5.0 and 3.8, 4.2; 1900 5.2, 6.0 and 5.5, 5.6;
 // 2100 7.0, 6.5 and 6.5, 6.2; 2800 7.9, 7.3 and 7.5, 7.3; 3300 8.5, 10.1 and 8.4, 9.5;
-// 4000 10.1, 11.0 and 10.1, 10.4; 7000 16.7, 17.7 and 16.7, 16.4; 16000 33.6, 34.7 and
-// 34.1, 34.0; 18000 37.6, 38.5 and 37.9, 38.1; 25500 51.3, 51.1 and 51.0, 51.9; 32000
-// 63.4, 63.1 and 63.0, 63.6.  8 + 1 heads, bf16 cache: 9216 22.0, 21.1.  32 + 8 heads,
-// fp32 tables: 2100 7.5, 7.8 and 7.0, 7.4; 2500 9.2, 8.4 and 8.5, 8.2; 3000 9.9, 10.9
-// and 9.6, 9.1; 3200 10.4, 11.4 and 9.8, 10.1; 9000 21.3, 24.2 and 22.0, 24.3; 16000
-// 34.6, 38.0 and 34.7, 38.0; 32768 66.0, 73.4 and 65.2, 68.5.
+// and, two with the positions first, 4050 10.4, 11.0 and 10.2, 10.0; 9000 20.9, 21.3 and
+// 21.0, 19.9; 16000 33.6, 34.6 and 34.0, 33.1; 20000 41.0, 41.2 and 41.2, 40.4; 25500
+// 51.3, 50.5 and 51.0, 51.1; 32768 64.6, 63.1 and 64.0, 62.1.  32 + 8 heads, fp32
+// tables: 2100 7.5, 7.8 and 7.0, 7.4; 2500 9.2, 8.4 and 8.5, 8.2; 3000 9.9, 10.9 and
+// 9.6, 9.1; 3200 10.4, 11.4 and 9.8, 10.1; 9000 21.3, 24.2 and 22.0, 24.3; 16000 34.6,
+// 38.0 and 34.7, 38.0; 32768 66.0, 73.4 and 65.2, 68.5.
 int rows_per_lane(int64_t one, bool fp8_cache, bool fp32_table) {
   if (one <= 2048) return 1;
   if (one <= (fp8_cache && fp32_table ? 2560 : 3072)) return 2;
@@ -746,8 +784,12 @@ int rows_per_lane(int64_t one, bool fp8_cache, bool fp32_table) {
 template <typename T, int CT>
 void launch_fast(const l20kv::Params &p, int cs_dtype, uint32_t rows_q, uint32_t rows_all, hipStream_t s) {
   const int64_t one = ((int64_t)rows_all + 4 * (64 / (p.d / 8)) - 1) / (4 * (64 / (p.d / 8)));
-  if (rows_per_lane(one, CT == 0, cs_dtype == 2) == 1) launch_fast_rows<T, CT, 1>(p, cs_dtype, rows_q, rows_all, s);
-  else launch_fast_rows<T, CT, 2>(p, cs_dtype, rows_q, rows_all, s);
+  if (rows_per_lane(one, CT == 0, cs_dtype == 2) == 1)
+    launch_fast_rows<T, CT, 1, false>(p, cs_dtype, rows_q, rows_all, s);
+  else if (one <= 3072)
+    launch_fast_rows<T, CT, 2, false>(p, cs_dtype, rows_q, rows_all, s);
+  else
+    launch_fast_rows<T, CT, 2, true>(p, cs_dtype, rows_q, rows_all, s);
 }
 
 template <typename T>
