@@ -1,4 +1,4 @@
-"""bench.py's output contract: one JSON line with the fields the driver reads.
+"""bench.py's output contract: one JSON line with the fields its readers take.
 
 The CPU test checks the one-GPU refusal; the GPU test runs a short headline
 bench in a child process (its own GPU context, a time limit) and checks every
