@@ -149,6 +149,8 @@ struct PartialParams {
   // count and the grid (n / d = umulhi(n, r); the host bounds n where the
   // quotient must be exact).
   unsigned int split_recip, heads_recip, grid_recip;
+  // pd_units only: log2 of the most waves that may share a unit.
+  int share_log2;
 };
 
 // ---------------------------------------------------------------------------
@@ -2009,8 +2011,11 @@ __global__ __launch_bounds__(64 * kFusedWaves) void pd_fp8_fused(PartialParams p
 // scan); workgroup i of G, one per CU, takes the i-th of G equal runs of them.
 // Each wave takes whole units of the run (wave w units w, w + 8, ...), or, with
 // few units, P = 2, 4 or 8 waves share one, each the p-th of P parts of its
-// blocks, and their states meet in LDS.  P is the largest whose waves fill at
-// most half of the chip's (all of them with two query tiles, whose blocks take
+// blocks, and their states meet in LDS.  P is the largest that leaves every part a
+// block of the longest unit (by the call's max_seq_len: a part without blocks only
+// adds to the meeting; 512-token splits, 208 x uniform 3-48 tokens, 2 KV heads 8.8
+// -> 7.6 us per call, 160 x 2-32 with two query tiles 10.8 -> 8.9) and whose waves fill
+// at most half of the chip's (all of them with two query tiles, whose blocks take
 // twice the arithmetic): beyond that the meeting costs more than the waves give
 // (fp8, 512-token splits, us per call with P = 1, 2, 4: 8 x 4096 tokens, 8 KV
 // heads, 512 units 22.2, 19.8, 20.5; 16 x 4096, 1024 units 28.3, 29.4; 9 x 4000,
@@ -2095,8 +2100,8 @@ __global__ __launch_bounds__(64 * kUnitWaves) void pd_units(PartialParams p) {
   }
   const int N = __builtin_amdgcn_readlane(incl, 63) * H;
   constexpr int kFill = NQT == 1 ? kUnitWaves / 2 : kUnitWaves;  // waves per workgroup that sharing may fill
-  int lp = 3;  // log2 P
-  while (lp > 0 && (((int64_t)N << lp) > (int64_t)G * kFill || (S >> lp) < kTok)) --lp;
+  int lp = p.share_log2;  // log2 P
+  while (lp > 0 && ((int64_t)N << lp) > (int64_t)G * kFill) --lp;
   const int P = 1 << lp;
   const int part = wave & (P - 1);
   const int step_units = kUnitWaves >> lp;
@@ -3015,7 +3020,7 @@ int device_cus() {
 }
 unsigned int recip32(int64_t d) { return d <= 1 ? 0u : (unsigned int)((((uint64_t)1 << 32) + d - 1) / d); }
 template <typename QT, int KT, int NQT, bool TREE>
-hipError_t launch_units_tiles(l20pd::PartialParams pp, int head_dim, int64_t units, hipStream_t stream) {
+hipError_t launch_units_tiles(l20pd::PartialParams pp, int head_dim, int64_t units, int longest, hipStream_t stream) {
   int64_t workgroups = std::min<int64_t>(units, device_cus());
   if (const char *cap = getenv("L20_PD_MAX_WORKGROUPS")) {  // as for the persistent kernel
     const long v = strtol(cap, nullptr, 10);
@@ -3025,6 +3030,8 @@ hipError_t launch_units_tiles(l20pd::PartialParams pp, int head_dim, int64_t uni
   pp.grid_recip = recip32(workgroups);
   pp.heads_recip = recip32(pp.num_kv_heads);
   pp.split_recip = recip32(pp.split_size);
+  pp.share_log2 = 3;
+  while (pp.share_log2 > 0 && (longest >> pp.share_log2) < (KT != 1 ? 32 : 16)) --pp.share_log2;
   // Blocks in flight per wave: two; one with two query tiles of fp8 caches (two
   // would spill) and, as in the persistent kernel, for fp8 splits of 1024 tokens, where
   // one is ahead with 5 to 8 units per CU of equal lengths (us per call with one and two,
@@ -3043,12 +3050,12 @@ hipError_t launch_units_tiles(l20pd::PartialParams pp, int head_dim, int64_t uni
   return hipGetLastError();
 }
 template <typename QT, int KT>
-hipError_t launch_units(const l20pd::PartialParams &pp, int head_dim, int nqt, int64_t units, hipStream_t stream) {
+hipError_t launch_units(const l20pd::PartialParams &pp, int head_dim, int nqt, int64_t units, int longest, hipStream_t stream) {
   if (nqt == 1)
-    return pp.tree ? launch_units_tiles<QT, KT, 1, true>(pp, head_dim, units, stream)
-                   : launch_units_tiles<QT, KT, 1, false>(pp, head_dim, units, stream);
-  return pp.tree ? launch_units_tiles<QT, KT, 2, true>(pp, head_dim, units, stream)
-                 : launch_units_tiles<QT, KT, 2, false>(pp, head_dim, units, stream);
+    return pp.tree ? launch_units_tiles<QT, KT, 1, true>(pp, head_dim, units, longest, stream)
+                   : launch_units_tiles<QT, KT, 1, false>(pp, head_dim, units, longest, stream);
+  return pp.tree ? launch_units_tiles<QT, KT, 2, true>(pp, head_dim, units, longest, stream)
+                 : launch_units_tiles<QT, KT, 2, false>(pp, head_dim, units, longest, stream);
 }
 // Whether the partial stage runs as pd_units rather than the persistent kernel:
 // wherever its batch (the lengths held per wave) and the exactness of its
@@ -3369,12 +3376,13 @@ int32_t run(const l20_pd_fp8_args *a, void *stream_ptr, int stages, int kinds) {
   } else if ((stages & kPartial) && units_fit(*a, pp, nqt, kv16)) {
     const int D = a->head_dim;
     const int64_t units = (int64_t)a->batch * a->num_kv_heads * pp.num_splits;
+    const int longest = std::min(a->split_size, a->max_seq_len);  // tokens of a unit, at most
     if (kv16)
-      e = bf16 ? launch_units<__bf16, 1>(pp, D, nqt, units, stream) : launch_units<_Float16, 1>(pp, D, nqt, units, stream);
+      e = bf16 ? launch_units<__bf16, 1>(pp, D, nqt, units, longest, stream) : launch_units<_Float16, 1>(pp, D, nqt, units, longest, stream);
     else if (e5m2)
-      e = bf16 ? launch_units<__bf16, 2>(pp, D, nqt, units, stream) : launch_units<_Float16, 2>(pp, D, nqt, units, stream);
+      e = bf16 ? launch_units<__bf16, 2>(pp, D, nqt, units, longest, stream) : launch_units<_Float16, 2>(pp, D, nqt, units, longest, stream);
     else
-      e = bf16 ? launch_units<__bf16, 0>(pp, D, nqt, units, stream) : launch_units<_Float16, 0>(pp, D, nqt, units, stream);
+      e = bf16 ? launch_units<__bf16, 0>(pp, D, nqt, units, longest, stream) : launch_units<_Float16, 0>(pp, D, nqt, units, longest, stream);
   } else if (stages & kPartial) {
     // Only the persistent kernel has a work queue: a call on another path must not
     // take a slot (and with it evict another stream's, or a captured launch's).

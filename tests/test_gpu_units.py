@@ -149,6 +149,34 @@ def test_units_shared_by_waves(case, waves, monkeypatch, no_queue):
         H.compare(*H.run_op16(inp, split, csr=csr), *H.run_oracle16(inp, csr=csr))
 
 
+@pytest.mark.parametrize("longest", [1, 15, 16, 17, 31, 32, 33, 63, 64, 65, 127, 128, 129])
+@pytest.mark.parametrize("case", [SHARED[0], SHARED[4], SHARED[8], SHARED[11]],
+                         ids=["fp8", "fp8_tree_2tiles", "bf16", "bf16_tree_2tiles"])
+def test_units_shared_no_finer_than_blocks(case, longest, kernels):
+    """One short split: the waves of a unit are as many as the longest sequence has whole
+    blocks (32 tokens with fp8 caches, 16 with 16-bit ones), on both sides of each step."""
+    _, hq, hkv, d, q_len, tree, cache, page, _ = case
+    lens = [max(q_len, x) for x in (longest, longest // 2, longest, longest - 1)] * 3
+    if cache == "e4m3fn":
+        inp = H.make_synthetic(len(lens), hq, hkv, d, lens, q_len=q_len, per_head=True, page=page, seed=longest,
+                               garbage_tail=True)
+    else:
+        inp = H.make_synthetic16(len(lens), hq, hkv, d, lens, dtype=torch.bfloat16, q_len=q_len, page=page,
+                                 seed=longest, garbage_tail=True)
+    if tree:
+        w = np.random.default_rng(longest).integers(0, 2**31, size=(len(lens), q_len), dtype=np.int64)
+        inp["tree_mask"] = torch.from_numpy(w.astype(np.int32)).cuda()
+    if cache == "e4m3fn":
+        (out, lse), (exp, exp_lse) = _run(inp, 512, torch.float32, kernels), H.run_oracle(inp)
+    else:
+        (out, lse), (exp, exp_lse) = H.run_op16(inp, 512), H.run_oracle16(inp)
+    # A row that sees one or two keys is as large as a value row (up to ~5, where half a
+    # bf16 step is 0.016): the output's own rounding, 2^-8 of it, is allowed on top.
+    err = np.abs(out.float().cpu().numpy() - exp)
+    assert (err <= H.OUT_ATOL + np.abs(exp) / 256).all(), err.max()
+    np.testing.assert_allclose(lse.cpu().numpy(), exp_lse, rtol=H.LSE_RTOL, atol=H.LSE_RTOL)
+
+
 @pytest.mark.parametrize("batch", [65, 256])
 def test_units_many_sequences(batch, monkeypatch, kernels):
     """Lanes hold two and four sequences' lengths."""
