@@ -228,7 +228,8 @@ int32_t l20_pd_single_launch(const l20_pd_fp8_args *args);
  * -(error code) when the arguments fail l20_pd_fp8_e4m3_check.  Host only, no
  * reference counterpart.  Of the calls that l20_pd_single_launch gives 0 for,
  * pd_units takes those of at most 256 sequences, except 16-bit caches beyond 16
- * units per CU and head_dim 64 beyond 32 (batch x num_kv_heads x splits). */
+ * units per CU, head_dim 64 beyond 32 (batch x num_kv_heads x splits) and some
+ * calls of short sequences of one split each. */
 int32_t l20_pd_partial_kernel(const l20_pd_fp8_args *args);
 
 /* Launches of the persistent partial kernel by this process so far: the calls

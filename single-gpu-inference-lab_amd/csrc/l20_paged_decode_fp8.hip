@@ -3057,19 +3057,41 @@ hipError_t launch_units(const l20pd::PartialParams &pp, int head_dim, int nqt, i
   return pp.tree ? launch_units_tiles<QT, KT, 2, true>(pp, head_dim, units, longest, stream)
                  : launch_units_tiles<QT, KT, 2, false>(pp, head_dim, units, longest, stream);
 }
-// Whether the partial stage runs as pd_units rather than the persistent kernel:
-// wherever its batch (the lengths held per wave) and the exactness of its
-// reciprocals allow, except large calls of the two kinds that measured faster on
-// the persistent kernel.  With 16-bit caches, beyond 16 units per CU at most (what
-// the host can see): 128 lognormal sequences, 4 KV heads 81.8 against 83.2 us per
-// call (8192 units at most), 64 of them 45.8 against 44.4 (4096).  At head_dim 64,
-// beyond 32: 200 x uniform to 3000, 8 KV heads 88.4 against 91.0 (9600), 100 of
-// them 53.6 against 46.5 (4800).  Within the bounds equal lengths can be faster on the
-// persistent kernel, but the host cannot tell them from ragged ones, which gain more
+// Short sequences of one split each, where the persistent kernel is ahead (it gives every
+// sequence a workgroup): us per call there and on pd_units, 512-token splits.
+// fp8, one query tile, 5 to 8 KV heads, a batch of at least 7/8 of the CUs: every wave of
+// pd_units has about one unit, and its loop of two blocks a turn computes one block too
+// many of a unit of an odd count.  256 x 5-84 tokens, 8 KV heads 13.4, 14.6; 6-96 13.6,
+// 14.7; 12-200 19.6, 20.8; 5 heads, 6-96 11.1, 12.2; but of an even count 8-128 15.5, 15.1,
+// and a batch of 200, 5 heads, 6-96 11.2, 10.3.  (With one block in flight, splits of 1024
+// tokens, a turn is one block.)
+// 16-bit caches, up to 4 KV heads, a batch of at least half the CUs: 200 x 4-64 tokens, 4
+// drafts of 16 / 2 heads 10.3, 13.8, of 28 / 4 heads 12.7, 14.3; one query tile only 17 to
+// 32 tokens of 2 heads (200 x 2-32 6.4, 7.3; 4-64 7.6, 7.7).
+bool short_split_fits(const l20_pd_fp8_args &a, int nqt, bool kv16, int64_t cus) {
+  const int64_t batch = a.batch, longest = a.max_seq_len;
+  if (a.max_seq_len > a.split_size || batch * a.num_kv_heads <= cus) return false;
+  if (kv16)
+    return 2 * batch >= cus && a.num_kv_heads <= (nqt == 2 ? 4 : 2) && longest > 16 &&
+           longest <= (nqt == 1 ? 32 : a.head_dim == 128 ? 128 : 64);
+  const int64_t blocks = (longest + 31) / 32;
+  return nqt == 1 && (a.head_dim == 64 || a.split_size < 1024) && 8 * batch >= 7 * cus && a.num_kv_heads >= 5 &&
+         a.num_kv_heads <= 8 && (blocks & 1) && blocks >= 3 && blocks <= 11;
+}
+
+// Whether the partial stage runs as pd_units rather than the persistent kernel: wherever
+// its batch (the lengths held per wave) and the exactness of its reciprocals allow,
+// except large calls of the two kinds that measured faster on the persistent kernel.
+// With 16-bit caches, beyond 16 units per CU at most (what the host can see): 128
+// lognormal sequences, 4 KV heads 81.8 against 83.2 us per call (8192 units at most), 64
+// of them 45.8 against 44.4 (4096).  At head_dim 64, beyond 32: 200 x uniform to 3000, 8
+// KV heads 88.4 against 91.0 (9600), 100 of them 53.6 against 46.5 (4800); and except
+// short sequences (short_split_fits).  Within the bounds equal lengths can be faster on
+// the persistent kernel, but the host cannot tell them from ragged ones, which gain more
 // (512-token splits, us per call on the persistent kernel and here, equal lengths,
-// uniform from an eighth, lognormal): 100 sequences to 2048 tokens, 2 KV heads 25.7 27.1,
-// 24.6 23.4, 23.8 17.0; 8 KV heads 83.5 85.7, 54.1 54.0, 36.3 31.2; 8 KV heads of 64
-// 61.5 66.4, 40.2 41.4, 31.4 25.5; 24 to 9000, 1024-token splits, 8 KV heads of 64
+// uniform from an eighth, lognormal): 100 sequences to 2048 tokens, 2 KV heads 25.7
+// 27.1, 24.6 23.4, 23.8 17.0; 8 KV heads 83.5 85.7, 54.1 54.0, 36.3 31.2; 8 KV heads of
+// 64 61.5 66.4, 40.2 41.4, 31.4 25.5; 24 to 9000, 1024-token splits, 8 KV heads of 64
 // 57.0 62.1, 49.7 34.6, 45.9 22.9.  L20_PD_UNITS=0/1 overrides the size rule (tests and
 // measurement).
 bool units_fit(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, int nqt, bool kv16) {
@@ -3080,8 +3102,8 @@ bool units_fit(const l20_pd_fp8_args &a, const l20pd::PartialParams &pp, int nqt
       ((int64_t)pp.l_cap + a.split_size) * a.split_size >= ((int64_t)1 << 32))
     return false;
   if (const char *env = getenv("L20_PD_UNITS")) return env[0] == '1';
-  const int64_t per_cu = kv16 ? 16 : a.head_dim == 64 ? 32 : INT64_MAX / 65536;
-  return units <= per_cu * device_cus();
+  const int64_t per_cu = kv16 ? 16 : a.head_dim == 64 ? 32 : INT64_MAX / 65536, cus = device_cus();
+  return units <= per_cu * cus && !short_split_fits(a, nqt, kv16, cus);
 }
 
 template <typename QT, int D, int WPP>

@@ -287,6 +287,38 @@ def test_partial_kernel_rule(monkeypatch):
         cabi.partial_kernel(a)
 
 
+def test_short_split_rule(monkeypatch):
+    """Short sequences of one split each keep the persistent kernel where it is ahead, on both
+    sides of each line (256 CUs here, no GPU)."""
+    for name in ("L20_PD_FUSED", "L20_PD_FUSED_SPLIT", "L20_PD_UNITS"):
+        monkeypatch.delenv(name, raising=False)
+
+    def kernel(batch, hq, hkv, longest, kv=cabi.L20_PD_KV_FP8_E4M3, q_len=1, split=512, d=128):
+        a = valid_args()
+        a.batch, a.num_q_heads, a.num_kv_heads, a.q_len, a.head_dim = batch, hq, hkv, q_len, d
+        a.max_seq_len, a.bt_stride_row, a.bt_max_pages, a.kv_dtype = longest, 64, 64, kv
+        _with_split(a, split)
+        return cabi.partial_kernel(a)
+
+    units, persistent = "pd_units", "pd_fp8_partial"
+    for longest, want in ((64, units), (65, persistent), (96, persistent), (97, units), (129, persistent),
+                          (352, persistent), (353, units), (416, units)):
+        assert kernel(224, 32, 8, longest) == want
+    assert kernel(223, 32, 8, 96) == units
+    assert kernel(224, 20, 5, 96) == persistent and kernel(224, 16, 4, 96) == units
+    assert kernel(224, 32, 16, 96) == units and kernel(224, 32, 8, 96, split=64) == units
+    assert kernel(224, 32, 8, 96, split=1024) == units and kernel(224, 32, 8, 96, split=1024, d=64) == persistent
+    assert kernel(224, 64, 8, 96, q_len=4) == units  # two query tiles: one block in flight
+    bf16 = cabi.L20_PD_KV_BF16
+    for longest, want in ((16, units), (17, persistent), (128, persistent), (129, units)):
+        assert kernel(200, 16, 2, longest, bf16, q_len=4) == want
+    assert kernel(200, 16, 2, 65, bf16, q_len=4, d=64) == units
+    assert kernel(200, 32, 4, 64, bf16, q_len=4) == persistent and kernel(200, 40, 5, 64, bf16, q_len=4) == units
+    assert kernel(127, 24, 3, 64, bf16, q_len=4) == units and kernel(128, 24, 3, 64, bf16, q_len=4) == persistent
+    assert kernel(200, 8, 2, 32, bf16) == persistent and kernel(200, 8, 2, 33, bf16) == units
+    assert kernel(200, 12, 3, 32, bf16) == units
+
+
 def test_split_mode_rule(monkeypatch):
     """l20_pd_single_launch returns 2 when the partial stage runs as the
     single-launch kernel's split mode (one workgroup per (split, sequence, KV
